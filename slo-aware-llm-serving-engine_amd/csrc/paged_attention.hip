@@ -224,26 +224,33 @@ struct Smem {
 // from fp32 overflow in the row sum) and O is rescaled only on those rare
 // tiles.  The result o / l is the same quantity as with an exact running max.
 constexpr float RESCALE_LOG2 = 8.0f;
+// Prefill: the largest probability sum of one lane's 8 keys of a half tile
+// (each probability is then at most this) before the column's offset moves.
+constexpr float PF_SUM_MAX = 512.0f;
 
 // Online softmax of one half tile (32 keys: score blocks sh[0], sh[1] hold key
 // rows kh + 16*mm + 4g + i) for the wavefront's NQT query columns.  Scores stay
-// unscaled until the exponent: max commutes with the positive factor
-// c = softmax_scale*log2(e), so e = exp2(c*s - c*m) is one FMA and one
-// v_exp_f32 per score; column reductions use v_permlane16/32_swap.  MASK
-// selects the boundary-tile path (keys past the tile's valid rows or causally
-// after the column).  SCALED (E4M3FN launches): scores take the keys' K scales
-// and probabilities their V scales from ks/vs (1.0 for tiles of bf16 rows),
-// without a per-score select.  Packs P^T into pb[nt] (the B operand of the half's PV
-// product) and returns in alpha[nt] the factor the accumulators must take
-// before that product; grow_any is set when any column's offset moved.
-// Branch-free for bf16 sources, so the compiler can interleave it with MFMA
-// work of the other half.
-template <int NQT, bool MASK, bool SCALED>
-__device__ __forceinline__ void softmax_half(f32x4 (&sh)[2][NQT], float (&m)[NQT], float (&l)[NQT], float (&alpha)[NQT],
-                                             bool& grow_any, bf16x8 (&pb)[NQT], float c,
-                                             const float* ks, const float* vs, int g, int ntok, int kh, int kv0,
-                                             int lim0) {
-  uint64_t grows = 0;
+// unscaled until the exponent: with ncm = -c*m, c = softmax_scale*log2(e),
+// e = exp2(c*s - c*m) is one FMA and one v_exp_f32 per score.  A tile's VALU
+// work is as long as its MFMA work, so the common path does nothing else:
+// no maximum is formed (a column whose offset is too small shows in its sums:
+// a lane's 8 probabilities add to more than PF_SUM_MAX, or to inf or NaN while
+// the offset is still unset, ncm = +inf), and l holds each lane's own sum,
+// added over the column's four lanes once per item.  Only then
+// does the wavefront take the branch that forms the columns' maxima, moves
+// the offsets of the columns that need it (all four lanes of a column decide
+// alike, whatever the wavefront's other columns do) and redoes the exponents.  MASK selects the boundary-tile path (keys past the tile's valid
+// rows or causally after the column).  SCALED (E4M3FN launches): scores take
+// the keys' K scales and probabilities their V scales from ks/vs (1.0 for
+// tiles of bf16 rows), without a per-score select.  Packs P^T into pb[nt] (the
+// B operand of the half's PV product); rescale(nt, a) multiplies column block
+// nt's accumulators by a before that product.
+template <int NQT, bool MASK, bool SCALED, typename Rescale>
+__device__ __forceinline__ void softmax_half(f32x4 (&sh)[2][NQT], float (&ncm)[NQT], float (&l)[NQT], bf16x8 (&pb)[NQT], float c, const float* ks, const float* vs, int g,
+                                             int ntok, int kh, int kv0, int lim0, Rescale&& rescale) {
+  f32x4 e[2][NQT];
+  float rs[NQT];
+  bool over = false;
 #pragma unroll
   for (int nt = 0; nt < NQT; ++nt) {
     if constexpr (SCALED) {
@@ -260,44 +267,66 @@ __device__ __forceinline__ void softmax_half(f32x4 (&sh)[2][NQT], float (&m)[NQT
           sh[mm][nt][i] = (tok < ntok && kv0 + tok <= lim) ? sh[mm][nt][i] : NEG_INF;
         }
     }
-    float mx = NEG_INF;
+    rs[nt] = 0.0f;
 #pragma unroll
     for (int mm = 0; mm < 2; ++mm)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sh[mm][nt][i]);
-    mx = col_max(mx);
-    const bool grow = c * (mx - m[nt]) > RESCALE_LOG2;  // false when both are -inf
-    const float mnew = grow ? mx : m[nt];
-    const float cm = mnew == NEG_INF ? 0.0f : c * mnew;
-    const float a = grow ? __builtin_amdgcn_exp2f(c * m[nt] - cm) : 1.0f;
-    float rs = 0.0f;
-#pragma unroll
-    for (int mm = 0; mm < 2; ++mm) {
-      f32x4 vsc = f32x4{1, 1, 1, 1};
-      if constexpr (SCALED) vsc = *reinterpret_cast<const f32x4*>(vs + kh + 16 * mm + 4 * g);
-#pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(sh[mm][nt][i], c, -cm));
-        rs += e;
-        // (Boundary tiles: the V scales of keys past the valid ones are
-        // whatever LDS holds there.)
-        const float v = MASK && SCALED ? (kh + 16 * mm + 4 * g + i < ntok ? vsc[i] : 0.0f) : vsc[i];
-        sh[mm][nt][i] = SCALED ? e * v : e;
+        e[mm][nt][i] = __builtin_amdgcn_exp2f(fmaf(sh[mm][nt][i], c, ncm[nt]));
+        rs[nt] += e[mm][nt][i];
+      }
+    over = over || !(rs[nt] <= PF_SUM_MAX);
+  }
+  if (__builtin_amdgcn_ballot_w64(over)) {
+#pragma unroll
+    for (int nt = 0; nt < NQT; ++nt) {
+      const bool grow = col_max(rs[nt] <= PF_SUM_MAX ? 0.0f : 1.0f) > 0.0f;
+      float mx = NEG_INF;
+#pragma unroll
+      for (int mm = 0; mm < 2; ++mm)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sh[mm][nt][i]);
+      mx = col_max(mx);
+      // (A column without a key yet keeps ncm = +inf and probabilities 0.)
+      const float next = grow && mx != NEG_INF ? fminf(ncm[nt], -c * mx) : ncm[nt];
+      const float nc = next == -NEG_INF ? 0.0f : next;
+      const float a = grow ? __builtin_amdgcn_exp2f(nc - ncm[nt]) : 1.0f;
+      rs[nt] = 0.0f;
+#pragma unroll
+      for (int mm = 0; mm < 2; ++mm)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          e[mm][nt][i] = __builtin_amdgcn_exp2f(fmaf(sh[mm][nt][i], c, nc));
+          rs[nt] += e[mm][nt][i];
+        }
+      l[nt] *= a;
+      ncm[nt] = next;
+      rescale(nt, a);
+    }
+  }
+#pragma unroll
+  for (int nt = 0; nt < NQT; ++nt) {
+    l[nt] += rs[nt];
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int mm = 0; mm < 2; ++mm) {
+        const f32x4 vsc = *reinterpret_cast<const f32x4*>(vs + kh + 16 * mm + 4 * g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          // (Boundary tiles: the V scales of keys past the valid ones are
+          // whatever LDS holds there.)
+          const float v = MASK ? (kh + 16 * mm + 4 * g + i < ntok ? vsc[i] : 0.0f) : vsc[i];
+          e[mm][nt][i] *= v;
+        }
       }
     }
-    rs = col_sum(rs);
-    l[nt] = l[nt] * a + rs;
-    m[nt] = mnew;
-    alpha[nt] = a;
-    grows |= __builtin_amdgcn_ballot_w64(grow);
     u32x4 w;
-    w.x = pack_bf16x2(sh[0][nt][0], sh[0][nt][1]);
-    w.y = pack_bf16x2(sh[0][nt][2], sh[0][nt][3]);
-    w.z = pack_bf16x2(sh[1][nt][0], sh[1][nt][1]);
-    w.w = pack_bf16x2(sh[1][nt][2], sh[1][nt][3]);
+    w.x = pack_bf16x2(e[0][nt][0], e[0][nt][1]);
+    w.y = pack_bf16x2(e[0][nt][2], e[0][nt][3]);
+    w.z = pack_bf16x2(e[1][nt][0], e[1][nt][1]);
+    w.w = pack_bf16x2(e[1][nt][2], e[1][nt][3]);
     pb[nt] = as_bf16x8(w);
   }
-  grow_any = grows != 0;
 }
 
 __device__ __forceinline__ int decode_len(const Params& p, int b) {
@@ -1482,10 +1511,10 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
   }
 
   f32x4 o[8][NQT];
-  float m[NQT], l[NQT];
+  float ncm[NQT], l[NQT];  // -c * the column's exponent offset, this lane's probability sum
 #pragma unroll
   for (int nt = 0; nt < NQT; ++nt) {
-    m[nt] = NEG_INF;
+    ncm[nt] = -NEG_INF;
     l[nt] = 0.0f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) o[dt][nt] = f32x4{0, 0, 0, 0};
@@ -1796,22 +1825,18 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj) kf[jj] = kread_h(1, jj);
       const int lim0 = q0 + n + prefix;
-      float a0[NQT], a1[NQT];
-      bool g0, g1;
       bf16x8 pb0[NQT], pb1[NQT];
+      auto rescale = [&](int nt, float a) {
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) o[dt][nt] *= a;
+      };
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj)
 #pragma unroll
         for (int nt = 0; nt < NQT; ++nt)
           s1[jj & 1][nt] = mfma16(as_bf16x8(kf[jj]), as_bf16x8(qv[nt][jj >> 1]), s1[jj & 1][nt]);
-      softmax_half<NQT, MASK, FP8>(s0, m, l, a0, g0, pb0, p.scale_log2, sm.u.pf.ks[buf], sm.u.pf.vs[buf], g, ntok,
-                            0, kv0, lim0);
-      if (g0) {
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-          for (int nt = 0; nt < NQT; ++nt) o[dt][nt] *= a0[nt];
-      }
+      softmax_half<NQT, MASK, FP8>(s0, ncm, l, pb0, p.scale_log2, sm.u.pf.ks[buf], sm.u.pf.vs[buf], g, ntok, 0,
+                                   kv0, lim0, rescale);
       bf16x8 vf[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) vf[i] = vread(i);
@@ -1819,14 +1844,8 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
       for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int nt = 0; nt < NQT; ++nt) o[i][nt] = mfma16(vf[i], pb0[nt], o[i][nt]);
-      softmax_half<NQT, MASK, FP8>(s1, m, l, a1, g1, pb1, p.scale_log2, sm.u.pf.ks[buf], sm.u.pf.vs[buf], g, ntok,
-                            32, kv0, lim0);
-      if (g1) {
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-          for (int nt = 0; nt < NQT; ++nt) o[dt][nt] *= a1[nt];
-      }
+      softmax_half<NQT, MASK, FP8>(s1, ncm, l, pb1, p.scale_log2, sm.u.pf.ks[buf], sm.u.pf.vs[buf], g, ntok, 32,
+                                   kv0, lim0, rescale);
 #pragma unroll
       for (int i = 0; i < 8; ++i) vf[i] = vread(8 + i);
 #pragma unroll
@@ -1870,10 +1889,14 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
     for (; kv0 < kstop; kv0 += TT, ++j) tile(T(), F(), kv0, j);
   }
 
+  // The column's probability sum: its four lanes' sums, added once.
+#pragma unroll
+  for (int nt = 0; nt < NQT; ++nt) l[nt] = col_sum(l[nt]);
+
   if constexpr (SPLITK) {
     if (two) {
       // Record layout (floats, NQT * PF_REC_FLOATS per item): O as
-      // [wave][nt][dt][lane] f32x4, then (m, l) as [wave][nt][lane] float2.
+      // [wave][nt][dt][lane] f32x4, then (ncm, l) as [wave][nt][lane] float2.
       constexpr int ML = 4 * NQT * 8 * 256;
       float* rec = p.partials + (size_t)item * (PF_REC_FLOATS * NQT);
       if (active) {
@@ -1884,7 +1907,7 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
             store16_agent(rec + (((wave * NQT + nt) * 8 + dt) * 64 + lane) * 4,
                           __builtin_bit_cast(u32x4, o[dt][nt]));
           store8_agent(rec + ML + ((wave * NQT + nt) * 64 + lane) * 2,
-                       u32x2{__float_as_uint(m[nt]), __float_as_uint(l[nt])});
+                       u32x2{__float_as_uint(ncm[nt]), __float_as_uint(l[nt])});
         }
       }
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // records stored before the ticket
@@ -1907,15 +1930,14 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
       const float* prec = p.partials + (size_t)(part ? item - pair : item + pair) * (PF_REC_FLOATS * NQT);
       // Merged in a fixed order (first half, then second), so the result's
       // rounding does not depend on which item arrived second.
-      const float c = p.scale_log2;
 #pragma unroll
       for (int nt = 0; nt < NQT; ++nt) {
         const float2 ml = load_partial2(prec + ML + ((wave * NQT + nt) * 64 + lane) * 2);
-        const float m0 = part ? ml.x : m[nt], m1 = part ? m[nt] : ml.x;
+        const float n0 = part ? ml.x : ncm[nt], n1 = part ? ncm[nt] : ml.x;
         const float l0 = part ? ml.y : l[nt], l1 = part ? l[nt] : ml.y;
-        const float mx = fmaxf(m0, m1);
-        const float w0 = m0 == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(c * (m0 - mx));
-        const float w1 = m1 == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(c * (m1 - mx));
+        const float nc = fminf(n0, n1);  // +inf: no key in that half
+        const float w0 = n0 == -NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(nc - n0);
+        const float w1 = n1 == -NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(nc - n1);
         l[nt] = fmaf(l1, w1, l0 * w0);
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {

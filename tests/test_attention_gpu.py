@@ -281,3 +281,23 @@ def test_merge_that_gives_up_is_reported_and_does_not_poison_the_next_launch(dev
     again, _ = case.run_gpu(device)
     check_workspaces()
     assert torch.equal(clean.view(torch.int16), again.view(torch.int16))
+
+
+@pytest.mark.parametrize("kv_fp8", [False, True])
+@pytest.mark.parametrize("rising", [False, True])
+def test_prefill_exponent_offsets_move(device, kv_fp8, rising):
+    # The prefill softmax moves a column's exponent offset only when a lane's
+    # probability sum exceeds its bound: keys whose scores rise by far more
+    # than 2^9 along the row move it many times (falling ones never after the
+    # first tile), in full, ragged and split rows, with and without a decode
+    # row beside them.  Peaked rows return single values, so V is scaled to
+    # |v| < 1.3: half a bf16 ulp there is 2^-8, and the probability's rounding
+    # adds at most 1.3 * 2^-9, within the gate's 2e-2.
+    for decode in ([], [40]):
+        case = Case(decode, [0, 300, 1200], [200, 97, 130], seed=21, kv_fp8=kv_fp8)
+        ramp = torch.linspace(0.1, 8.0, case.k.shape[0])[:, None, None]
+        case.k = (case.k.float() * (ramp if rising else ramp.flip(0))).to(torch.bfloat16)
+        case.q = (case.q.float() * 3).to(torch.bfloat16)
+        case.v = (case.v.float() / 4).to(torch.bfloat16)
+        case.old_v = [(v.float() / 4).to(torch.bfloat16) for v in case.old_v]
+        _check(case, device)
