@@ -150,12 +150,16 @@ __device__ __forceinline__ void atomic_add_noret(void* p, uint32_t v) {
   asm volatile("global_atomic_add %0, %1, off" ::"v"(p), "v"(v) : "memory");
 }
 // Stores: agent-scope (write-through to the coherence point) for split-K
-// partials, plain for outputs.
+// partials, plain for outputs.  A store of more than 64 bits per lane reads its
+// data after it issues: the registers may be written again only two wait
+// states later, which the compiler does not know of a store written in asm
+// (records lost lanes 12-15 of an element when the next instruction reused
+// its register).
 __device__ __forceinline__ void store16_agent(void* p, const u32x4& v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 __device__ __forceinline__ void store16(void* p, const u32x4& v) {
-  asm volatile("global_store_dwordx4 %0, %1, off" ::"v"(p), "v"(v) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 __device__ __forceinline__ void store8(void* p, const u32x2& v) {
   asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(p), "v"(v) : "memory");
