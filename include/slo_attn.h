@@ -40,6 +40,10 @@ enum {
 enum { SLO_KV_BF16 = 0, SLO_KV_FP8_E4M3FN = 1 };
 
 enum { SLO_PHASE_DECODE = 1, SLO_PHASE_PREFILL = 2, SLO_PHASE_ALL = 3 };
+/* Or-ed into phases: the rows of new_k / new_v may lie any multiple of 8
+ * elements (at least num_kv_heads * head_dim) apart, as views of a fused
+ * projection's output do.  Launches without prefill rows only. */
+enum { SLO_NEW_ROWS_STRIDED = 256 };
 
 /* Smallest FP8 scale: a power of two, so a scale is always a normal fp32 and
  * no denormal arithmetic can change a code. */
@@ -190,7 +194,7 @@ typedef struct slo_paged_attention_args {
 
   void* workspace;                /* zero-filled once at allocation */
   size_t workspace_bytes;
-  int32_t phases;                 /* SLO_PHASE_* mask */
+  int32_t phases;                 /* SLO_PHASE_* mask, optionally | SLO_NEW_ROWS_STRIDED */
 
   /* Optional KV write in the same launch, the store of
    * forward_mixed / Attention.forward (nanovllm/layers/mixed_attention.py:
@@ -199,7 +203,7 @@ typedef struct slo_paged_attention_args {
    * slo_store_kvcache with store_scale_floor, and at most 8 query heads per
    * kv head).  When store_slot_mapping is not NULL, new row t of new_k/new_v
    * ([num_new_rows == num_q_rows, num_kv_heads, head_dim] bf16, contiguous:
-   * row stride num_kv_heads * head_dim, 16-byte aligned; decode rows' tokens first,
+   * row stride num_kv_heads * head_dim (see SLO_NEW_ROWS_STRIDED), 16-byte aligned; decode rows' tokens first,
    * then the prefill rows' tokens in cu_seqlens_q order) is written to pool
    * slot store_slot_mapping[t] (slots < 0 or past the pool are skipped), and
    * the launch reads the step's new tokens from new_k/new_v instead of the

@@ -2573,8 +2573,13 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
     if (!a->k_cache || !a->v_cache || a->num_blocks <= 0 || a->block_size <= 0)
       return fail(SLO_ERR_INVALID, "paged_attention: the KV write needs the pool");
     const int64_t row = (int64_t)a->num_kv_heads * HD;
-    if (!a->new_k || !a->new_v || a->num_new_rows != a->num_q_rows || a->new_k_row_stride != row ||
-        a->new_v_row_stride != row || (reinterpret_cast<uintptr_t>(a->new_k) % 16) ||
+    // Launches without prefill rows address each new row by its own stride, so
+    // views of a fused projection's output fold as well (prefill tiles of new
+    // tokens take the pool's row length).
+    const bool strided = (a->phases & SLO_NEW_ROWS_STRIDED) && !do_pf;
+    auto bad_stride = [&](int64_t st) { return strided ? st < row || st % 8 : st != row; };
+    if (!a->new_k || !a->new_v || a->num_new_rows != a->num_q_rows || bad_stride(a->new_k_row_stride) ||
+        bad_stride(a->new_v_row_stride) || (reinterpret_cast<uintptr_t>(a->new_k) % 16) ||
         (reinterpret_cast<uintptr_t>(a->new_v) % 16))
       return fail(SLO_ERR_INVALID,
                   "paged_attention: new K/V must be contiguous 16-byte aligned bf16 rows, one per query row");

@@ -14,7 +14,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .ops import check_store, foldable, paged_attention, store_kvcache
+from .ops import check_store, foldable, foldable_strided, paged_attention, store_kvcache
 
 
 @dataclass
@@ -57,8 +57,13 @@ def forward_mixed(q, k, v, k_cache, v_cache, context, scale, store_fn,
     # decode rows and two chunks, one after a 1,024-token prefix: 108 against
     # 72 us), and cold rows run in the E4M3FN instantiation, which spills
     # registers (4 cold rows: 134 against 107 us).
-    fold = (store_fn is store_kvcache and phases == _lib.PHASE_ALL and foldable(k, v)
-            and (k_scale is None or (q.shape[1] <= 8 * k.shape[1] and not meta.num_prefill_tokens)))
+    # Pure decode steps also fold rows that are views of the QKV projection.
+    decode_only = not meta.num_prefill_tokens
+    fold = (store_fn is store_kvcache and phases == _lib.PHASE_ALL
+            and (foldable_strided(k, v) if decode_only else foldable(k, v))
+            and (k_scale is None or (q.shape[1] <= 8 * k.shape[1] and decode_only)))
+    if fold and decode_only:
+        phases |= _lib.NEW_ROWS_STRIDED
     if fold:
         check_store(k, v, k_cache, v_cache, context.slot_mapping, k_scale, v_scale)
     elif k_scale is None:

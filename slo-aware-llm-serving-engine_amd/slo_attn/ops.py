@@ -97,6 +97,18 @@ def foldable(key: torch.Tensor, value: torch.Tensor) -> bool:
             and key.stride(1) == key.shape[2] and value.stride(1) == value.shape[2])
 
 
+def foldable_strided(key: torch.Tensor, value: torch.Tensor) -> bool:
+    """Whether a launch without prefill rows can carry the KV write of these
+    new rows (``_lib.NEW_ROWS_STRIDED``): bf16 ``[N, num_kv_heads, head_dim]``
+    rows of contiguous heads on 16-byte boundaries, such as the K and V views
+    of a fused QKV projection's output."""
+    if key.dim() != 3 or key.dtype != torch.bfloat16 or value.dtype != torch.bfloat16:
+        return False
+    row, d = key.shape[1] * key.shape[2], key.shape[2]
+    return all(t.stride(2) == 1 and t.stride(1) == d and t.stride(0) >= row and t.stride(0) % 8 == 0
+               and t.data_ptr() % 16 == 0 for t in (key, value))
+
+
 def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, slot_mapping: torch.Tensor,
                   k_scale: torch.Tensor | None = None, v_scale: torch.Tensor | None = None,

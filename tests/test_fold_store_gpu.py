@@ -297,3 +297,68 @@ def test_folded_store_with_prefixes_inside_a_key_tile(device, prefixes):
     torch.cuda.synchronize()
     assert torch.equal(got2.view(torch.int16), ref2.view(torch.int16))
     assert torch.equal(kc3.view(torch.int16), kc2.view(torch.int16))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("rows,hi,hkv", [(1, 700, 8), (5, 300, 4), (40, 4000, 8), (150, 4096, 8)])
+def test_decode_folds_views_of_the_qkv_projection(device, fp8, rows, hi, hkv):
+    # Decode steps fold K/V rows that are views of the fused projection's
+    # output (row stride larger than a pool row), bf16 and E4M3FN, in the
+    # direct kernel and (150 long rows) the work lists: output and pool bytes
+    # of the store kernel followed by the attention launch, through
+    # Attention.forward's V0 decode branch and through forward_mixed.
+    g = torch.Generator().manual_seed(rows + hkv)
+    hq, dh, bs = 4 * hkv, 128, 256
+    lens = torch.randint(1, hi + 1, (rows,), generator=g).tolist()
+    lens[0] = hi
+    per = [(n + bs - 1) // bs for n in lens]
+    nblk, width = sum(per) + 1, max(per)
+    perm = torch.randperm(nblk, generator=g).tolist()
+    tables, at = [], 0
+    for n in per:
+        tables.append(perm[at:at + n])
+        at += n
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)  # noqa: E731
+    slots = i32([t[(n - 1) // bs] * bs + (n - 1) % bs for t, n in zip(tables, lens)])
+    padded, dl = i32([t + [-1] * (width - len(t)) for t in tables]), i32(lens)
+    qkv = torch.randn(rows, (hq + 2 * hkv) * dh, generator=g).to(torch.bfloat16).to(device)
+    q, k, v = (t.view(rows, -1, dh) for t in qkv.split([hq * dh, hkv * dh, hkv * dh], -1))
+    q = q.contiguous()
+    reserve_workspace(device, rows, width * bs, hq, hkv, dh)
+    base = torch.randn(2, nblk, bs, hkv, dh, generator=g).to(torch.bfloat16).to(device)
+
+    def pools():
+        if not fp8:
+            return [base[0].clone(), base[1].clone()]
+        p = [torch.empty(nblk, bs, hkv, dh, dtype=torch.uint8, device=device) for _ in range(2)]
+        s = [torch.empty(nblk, bs, hkv, device=device) for _ in range(2)]
+        every = torch.arange(nblk * bs, dtype=torch.int32, device=device)
+        store_kvcache(base[0].view(-1, hkv, dh), base[1].view(-1, hkv, dh), *p, every, *s)
+        return p + s
+
+    ctx = SimpleNamespace(mixed=MixedAttentionContext(rows, 0, dl, padded, None, None, None, 0, 0),
+                          slot_mapping=slots)
+    ref_pools, got_pools, v0_pools = pools(), pools(), pools()
+    ref = forward_mixed(q, k, v, ref_pools[0], ref_pools[1], ctx, dh ** -0.5, _two_launch_store, *ref_pools[2:])
+    got = forward_mixed(q, k, v, got_pools[0], got_pools[1], ctx, dh ** -0.5, store_kvcache, *got_pools[2:])
+    attn = Attention(hq, dh, dh ** -0.5, hkv)
+    attn.k_cache, attn.v_cache = v0_pools[:2]
+    if fp8:
+        attn.k_scale, attn.v_scale = v0_pools[2:]
+    set_context(False, slot_mapping=slots, context_lens=dl, block_tables=padded)
+    v0 = attn(q, k, v).squeeze(1)
+    reset_context()
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    assert torch.equal(v0.view(torch.int16), ref.view(torch.int16))
+    for a_, b_, c_ in zip(ref_pools, got_pools, v0_pools):
+        assert torch.equal(a_.view(torch.uint8), b_.view(torch.uint8))
+        assert torch.equal(a_.view(torch.uint8), c_.view(torch.uint8))
+    # Without the flag for strided rows the launch refuses them, as it does
+    # beside prefill rows.
+    if rows > 1:
+        with pytest.raises(RuntimeError):
+            paged_attention(q, got_pools[0], got_pools[1], dh ** -0.5, num_kv_heads=hkv,
+                            k_scale=got_pools[2] if fp8 else None, v_scale=got_pools[3] if fp8 else None,
+                            num_decode=rows, decode_lens=dl, decode_tables=padded, store_slot_mapping=slots,
+                            new_k=k, new_v=v)
