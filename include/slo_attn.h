@@ -42,7 +42,8 @@ enum { SLO_KV_BF16 = 0, SLO_KV_FP8_E4M3FN = 1 };
 enum { SLO_PHASE_DECODE = 1, SLO_PHASE_PREFILL = 2, SLO_PHASE_ALL = 3 };
 /* Or-ed into phases: the rows of new_k / new_v may lie any multiple of 8
  * elements (at least num_kv_heads * head_dim) apart, as views of a fused
- * projection's output do.  Launches without prefill rows only. */
+ * projection's output do.  Only for launches without prefill rows, or with
+ * num_decode 0 and prefill_tables NULL. */
 enum { SLO_NEW_ROWS_STRIDED = 256 };
 
 /* Smallest FP8 scale: a power of two, so a scale is always a normal fp32 and
@@ -212,9 +213,10 @@ typedef struct slo_paged_attention_args {
    * num_decode + cu_q[r] + j - (Lk - Lq).  The result equals the separate
    * store followed by this launch, bit for bit; no slot written by the launch
    * may be read through a table by it except as such a new token.  Launches
-   * without decode rows, and E4M3FN launches with prefill rows, make that
-   * order themselves: the store kernel, then the attention launch (two
-   * kernels on `stream`, the same bytes and outputs). */
+   * without decode rows whose prefill rows have tables, and E4M3FN launches
+   * with decode and prefill rows, make that order themselves: the store
+   * kernel, then the attention launch (two kernels on `stream`, the same
+   * bytes and outputs). */
   const int32_t* store_slot_mapping;  /* [num_new_rows] or NULL */
   const void* new_k;
   int64_t new_k_row_stride;

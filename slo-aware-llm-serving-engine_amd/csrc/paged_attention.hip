@@ -171,6 +171,7 @@ struct Params {
   int32_t nnew;
   int64_t num_slots;
   float scale_floor;  // E4M3FN pools with the KV write folded in: the store's scale_floor
+  int32_t store_fp8;  // prefill-only launches with the KV write: the pool is E4M3FN
   // How long a split-K merge task waits for its chunks before it gives up
   // (s_memrealtime ticks).
   int64_t merge_wait_ticks;
@@ -1019,6 +1020,48 @@ __device__ __forceinline__ void store_new_rows(const Params& p, int64_t first, i
   }
 }
 
+// KV write of new rows [t0, t0 + n) of kv head h, by a prefill-only launch
+// that reads no pool (cold rows): 16 + 16 pieces of 16 bytes a row (K, V).
+__device__ __forceinline__ void store_head_rows(const Params& p, int64_t t0, int n, int h, int tid) {
+  n = (int)min((int64_t)n, (int64_t)p.nnew - t0);
+  for (int i0 = 0; i0 < 32 * n; i0 += 4 * NT) {
+    u32x4 x[4];
+    int64_t slot[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = i0 + j * NT + tid;
+      slot[j] = -1;
+      x[j] = u32x4{0, 0, 0, 0};
+      if (i < 32 * n) {
+        const int64_t t = t0 + (i >> 5);
+        x[j] = ld16(((i & 16) ? p.nv + t * p.nv_stride : p.nk + t * p.nk_stride) + h * HD + 8 * (i & 15));
+        slot[j] = p.sslots[t];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bool isv = tid & 16;  // (NT is a multiple of 32)
+      const int64_t vec = slot[j] * p.hkv + h;
+      uint8_t* base = static_cast<uint8_t*>(const_cast<void*>(isv ? p.v_cache : p.k_cache));
+      if (p.store_fp8) {
+        float f[8], sc;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          f[2 * k] = bf16_bits_to_f32(x[j][k] & 0xffffu);
+          f[2 * k + 1] = bf16_bits_to_f32(x[j][k] >> 16);
+        }
+        const u32x2 codes = e4m3_encode8<HD / 8>(f, p.scale_floor, sc);
+        if (slot[j] < 0 || slot[j] >= p.num_slots) continue;
+        *reinterpret_cast<u32x2*>(base + vec * HD + 8 * (tid & 15)) = codes;
+        if ((tid & 15) == 0) const_cast<float*>(isv ? p.v_scale : p.k_scale)[vec] = sc;
+      } else {
+        if (slot[j] < 0 || slot[j] >= p.num_slots) continue;
+        st16(base + vec * ROWB + 16 * (tid & 15), x[j]);
+      }
+    }
+  }
+}
+
 // Tail tasks, taken by each workgroup once its items are done: first the KV
 // write of the launch's new tokens (when the launch carries it), then the
 // split-K merges.  Store task i of list l writes new rows [4g, 4g + 4) for
@@ -1462,7 +1505,9 @@ __global__ void __launch_bounds__(NT, 2) decode_direct_kernel(Params p, int nch_
 // (local index ((block * 2 + part) * hkv + h) * HG + hg, global `item`); each
 // writes (O, m, l) of its range as a record, and the one that arrives second
 // on the pair's ticket merges both and writes the output.
-template <bool FP8, int NQT, bool FOLD, bool SPLITK = false>
+// SRC: where the keys come from, when the launch's shape says so.
+enum PfSource : int { SRC_ANY = 0, SRC_POOL = 1, SRC_ROWS = 2 };
+template <bool FP8, int NQT, bool FOLD, bool SPLITK = false, int SRC = SRC_ANY>
 __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* st1, int r, int local, int tid,
                              int item = 0, bool split = false) {
   static_assert(!(FP8 && FOLD), "E4M3FN launches with prefill rows run the store kernel first");
@@ -1480,7 +1525,7 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
   const PfRow geo = pf_row(p, r);
   const int q_start = geo.q_start, Lq = geo.Lq, k_start = geo.k_start, Lk = geo.Lk;
   const int prefix = geo.prefix;  // bottom-right causal alignment
-  const bool paged = p.ptab != nullptr;
+  const bool paged = SRC == SRC_POOL || (SRC == SRC_ANY && p.ptab != nullptr);
 
   const int nqb = (Lq + BQ - 1) / BQ;
   const int q0 = (nqb - 1 - qb_rev) * BQ;  // heaviest blocks are pulled first
@@ -1985,9 +2030,12 @@ __device__ void prefill_item(const Params& p, Smem& sm, uint8_t* st0, uint8_t* s
 // register-allocated without the code of paths the launch cannot take.
 enum Mode : int {
   MODE_MIXED = 0,    // decode and prefill rows; prefill in 32-position blocks
-  MODE_PREFILL = 1,  // prefill rows only; block size chosen per launch
+  MODE_PREFILL = 1,  // prefill rows only, keys from the pool; block size chosen per launch
   MODE_DECODE = 2,   // decode rows only
+  MODE_COLD = 3,     // as MODE_PREFILL, keys from the new rows only; may carry the KV write
 };
+
+constexpr int MODES = 4;
 
 // FOLD: the launch carries the KV write of the step's new tokens (bf16
 // pools): prefill tiles read new tokens from the new rows, and the tail tasks
@@ -1995,7 +2043,11 @@ enum Mode : int {
 // the prefill tile loop's smaller register footprint.
 template <bool FP8, int MODE, bool FOLD = false>
 __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
-  constexpr bool HAS_DEC = MODE != MODE_PREFILL;
+  constexpr bool PF_ONLY = MODE == MODE_PREFILL || MODE == MODE_COLD;
+  constexpr bool HAS_DEC = !PF_ONLY;
+  // (The bf16 MODE_PREFILL instantiation spilled registers with the source
+  // known; the E4M3FN one went from 256 to 239.)
+  constexpr int SRC = MODE == MODE_PREFILL && FP8 ? SRC_POOL : MODE == MODE_COLD ? SRC_ROWS : SRC_ANY;
   constexpr bool HAS_PF = MODE != MODE_DECODE;
   __shared__ Smem sm;
   __shared__ __attribute__((aligned(16))) uint8_t stage0[STAGE_BYTES];
@@ -2003,7 +2055,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
   // decode: Q of the current and next item
   __shared__ __attribute__((aligned(16))) uint8_t qbuf[HAS_DEC ? 2 * QBUF : 16];
   // Prefill-only launches: the ranked units and the rows' geometry.
-  constexpr bool PF_SORT = MODE == MODE_PREFILL;
+  constexpr bool PF_SORT = PF_ONLY;
   __shared__ uint32_t pf_units[PF_SORT ? PF_SORT_UNITS : 1];
   __shared__ int4 pf_geo[PF_SORT ? PF_SORT_ROWS : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2071,7 +2123,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
       w += __shfl_xor(w, d, 64);
       tm = max(tm, __shfl_xor(tm, d, 64));
       dn += __shfl_xor(dn, d, 64);
-      if constexpr (MODE == MODE_PREFILL && !FOLD) tu = max(tu, __shfl_xor(tu, d, 64));
+      if constexpr (PF_ONLY && !FOLD) tu = max(tu, __shfl_xor(tu, d, 64));
     }
     if (lane == 0) {
       sm.wsum[wave] = w;
@@ -2089,7 +2141,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
       dt += sm.dsum[i];
       tunsplit = max(tunsplit, sm.wumax[i]);
     }
-    pf_long = MODE == MODE_PREFILL && (int64_t)tmax * gridDim.x > 2 * wt;
+    pf_long = PF_ONLY && (int64_t)tmax * gridDim.x > 2 * wt;
     if (pf_long) {
       // Rows that split their keys in two (below) halve their longest items
       // already, and take 32-position blocks, whose tiles cost half the LDS
@@ -2138,7 +2190,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
       // 256-4096 tokens with two 512-token chunks 65.8 -> 66.5 us, while 64
       // rows of 512-4096 with one 1,024-token chunk went 146.4 -> 137.6 us.
       sm.kv_nt = MODE != MODE_MIXED || 4 * dt * p.hkv >= 4 * wt;
-      sm.pf_split_thr = MODE == MODE_PREFILL ? (int)max((int64_t)16, 2 * wt / gridDim.x) : (1 << 30);
+      sm.pf_split_thr = PF_ONLY ? (int)max((int64_t)16, 2 * wt / gridDim.x) : (1 << 30);
     }
     __syncthreads();
   }
@@ -2149,7 +2201,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
   // two key ranges per item, merged by the range that finishes second, when
   // every item of the launch has a record slot (a ticket and pf_split_bytes
   // of records); such a row otherwise sets the launch's length alone.
-  if constexpr (MODE == MODE_PREFILL) {
+  if constexpr (PF_ONLY) {
     int base_c = 0, extra_c = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -2187,7 +2239,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
   int local_sum = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const bool sp = MODE == MODE_PREFILL && r0 + i < p.np && pf_splits(p, r0 + i, tmr[i], sm.pf_split_thr);
+    const bool sp = PF_ONLY && r0 + i < p.np && pf_splits(p, r0 + i, tmr[i], sm.pf_split_thr);
     const bool alt = r0 + i < p.np ? ((bq == 16 && !(sp && !FOLD)) || tmr[i] > sm.split_tiles)
                                    : dchunk == d_chunk_min<FP8>();
     cnt[i] = cnt_a[i] + (alt ? cnt_d[i] : 0);
@@ -2347,7 +2399,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
       const int ltid = tid + sm.salt;
       if (HAS_PF && r < p.np) {
         const int item = list + (int)rel * nlist;
-        if constexpr (MODE == MODE_PREFILL) {
+        if constexpr (PF_ONLY) {
           bool sp = false;
           {
             int wr = 0, tr = 0;
@@ -2360,11 +2412,11 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
           const int lr = sorted ? (int)(pf_units[item / per_unit] & 0xffffu) * per_unit + item % per_unit
                                 : item - sm.off[r];
           if (sp) {
-            if constexpr (!FOLD) prefill_item<FP8, 2, FOLD, true>(p, sm, stage0, stage1, r, lr, ltid, item, true);
-            else prefill_item<FP8, 1, FOLD, true>(p, sm, stage0, stage1, r, lr, ltid, item, true);
+            if constexpr (!FOLD) prefill_item<FP8, 2, FOLD, true, SRC>(p, sm, stage0, stage1, r, lr, ltid, item, true);
+            else prefill_item<FP8, 1, FOLD, true, SRC>(p, sm, stage0, stage1, r, lr, ltid, item, true);
           }
-          else if (bq == 16) prefill_item<FP8, 1, FOLD>(p, sm, stage0, stage1, r, lr, ltid);
-          else prefill_item<FP8, 2, FOLD>(p, sm, stage0, stage1, r, lr, ltid);
+          else if (bq == 16) prefill_item<FP8, 1, FOLD, false, SRC>(p, sm, stage0, stage1, r, lr, ltid);
+          else prefill_item<FP8, 2, FOLD, false, SRC>(p, sm, stage0, stage1, r, lr, ltid);
         } else if constexpr (HAS_PF) {
           // The row's items are 16-position blocks exactly when the item
           // counts above took them so (tmr > split_tiles, E4M3FN launches).
@@ -2379,6 +2431,26 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
         // first.
         uint32_t next = 0;
         if (tid == 0) next = atomicAdd(ctr, 1u) - base;
+        if constexpr (MODE == MODE_COLD) {
+          // A launch of cold rows that carries the KV write reads no pool, so
+          // each item writes its block's new tokens of its kv head, beside
+          // the fetch's round trip and the other workgroups' products (four
+          // cold rows of 346-1,813 tokens: 79.0 -> 76.6 us a layer against
+          // the store kernel's own launch of 9 us).
+          if (p.nnew > 0) {
+            int wr = 0, tr = 0;
+            pf_work(p, r, wr, tr);
+            const bool sp = pf_splits(p, r, tr, sm.pf_split_thr);
+            const int lr = sorted ? (int)(pf_units[item / per_unit] & 0xffffu) * per_unit + item % per_unit
+                                  : item - sm.off[r];
+            const int blk = sp || bq == 32 ? 32 : 16;
+            const int t = lr / p.HG, u = t / p.hkv;
+            const int start = p.cu_q[r], Lq = p.cu_q[r + 1] - start;
+            const int q0 = ((Lq + blk - 1) / blk - 1 - (sp ? u >> 1 : u)) * blk;
+            if (lr % p.HG == 0 && !(sp && (u & 1)) && q0 >= 0)
+              store_head_rows(p, (int64_t)p.q_off_prefill + start + q0, min(blk, Lq - q0), t % p.hkv, ltid);
+          }
+        }
         rel = advance(next);
         r = resolve(rel);
         continue;
@@ -2398,6 +2470,15 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
     __syncthreads();
   }
   tail_tasks<FP8, FOLD>(p, sm, list, nlist, decode_base, dchunk, tid);
+  if constexpr (MODE == MODE_COLD) {
+    // New rows outside every prefill row.
+    const int head = p.nnew > 0 ? min(max(p.cu_q[0], 0), p.nnew) : 0;
+    const int tail = p.nnew > 0 ? min(max(p.cu_q[p.np], 0), p.nnew) : 0;
+    for (int x = blockIdx.x; x < (head + p.nnew - tail) * p.hkv; x += gridDim.x) {
+      const int t = x / p.hkv;
+      store_head_rows(p, t < head ? t : tail + t - head, 1, x % p.hkv, tid);
+    }
+  }
 
   // Rows that belong to no decode or prefill row (the capacity padding of a
   // captured step) get zeros, so every output row is defined.
@@ -2416,15 +2497,19 @@ using AttnKernel = void (*)(Params);
 
 // The instantiations, indexed [fold][fp8][mode].
 AttnKernel attn_kernel(bool fold, bool fp8, int mode) {
-  static const AttnKernel table[2][2][3] = {
+  static const AttnKernel table[2][2][MODES] = {
+      // (A launch of cold rows reads nothing from an E4M3FN pool.)
       {{paged_attention_kernel<false, MODE_MIXED>, paged_attention_kernel<false, MODE_PREFILL>,
-        paged_attention_kernel<false, MODE_DECODE>},
+        paged_attention_kernel<false, MODE_DECODE>, paged_attention_kernel<false, MODE_COLD>},
        {paged_attention_kernel<true, MODE_MIXED>, paged_attention_kernel<true, MODE_PREFILL>,
-        paged_attention_kernel<true, MODE_DECODE>}},
-      // Prefill-only launches and E4M3FN launches with prefill rows never
-      // carry the KV write (launch_attention runs the store kernel first).
-      {{paged_attention_kernel<false, MODE_MIXED, true>, nullptr, paged_attention_kernel<false, MODE_DECODE, true>},
-       {nullptr, nullptr, paged_attention_kernel<true, MODE_DECODE, true>}},
+        paged_attention_kernel<true, MODE_DECODE>, nullptr}},
+      // Prefill-only launches of rows with tables and E4M3FN launches with
+      // decode and prefill rows never carry the KV write (launch_attention
+      // runs the store kernel first); launches of cold rows carry it in their
+      // own instantiation, FOLD or not.
+      {{paged_attention_kernel<false, MODE_MIXED, true>, nullptr, paged_attention_kernel<false, MODE_DECODE, true>,
+        nullptr},
+       {nullptr, nullptr, paged_attention_kernel<true, MODE_DECODE, true>, nullptr}},
   };
   return table[fold ? 1 : 0][fp8 ? 1 : 0][mode];
 }
@@ -2450,7 +2535,7 @@ constexpr int DIRECT_CHUNK_MAX = 1024;  // tokens
 struct DeviceShape {
   int cus = 0;
   int wallclock_khz = 0;  // s_memrealtime rate
-  int wg_per_cu[2][2][3] = {};
+  int wg_per_cu[2][2][MODES] = {};
   int wg_direct[2] = {};  // decode_direct_kernel (without the KV write), by pool format
 };
 
@@ -2469,7 +2554,7 @@ int device_shape(DeviceShape* out) {
     if (s.wallclock_khz <= 0) s.wallclock_khz = 100000;
     for (int fold = 0; fold < 2; ++fold)
       for (int fp8 = 0; fp8 < 2; ++fp8)
-        for (int mode = 0; mode < 3; ++mode) {
+        for (int mode = 0; mode < MODES; ++mode) {
           const AttnKernel k = attn_kernel(fold, fp8, mode);
           if (!k) continue;
           int n = 0;
@@ -2575,6 +2660,9 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
   // for the step; four cold rows of 267-1,843 tokens 91.1 -> 90.1 us), while
   // the mixed launch gains from the fold (65.5 against 70.6 us).
   const bool fold = store && do_dec && !(fp8 && do_pf);
+  // Prefill rows without tables read the contiguous K/V only: the launch's
+  // items write the new rows to the pool (store_head_rows).
+  const bool cold = store && do_pf && a->num_decode == 0 && !a->prefill_tables;
   if (store) {
     if (fp8 && !(a->store_scale_floor > 0.0f))
       return fail(SLO_ERR_INVALID, "paged_attention: the E4M3FN KV write needs store_scale_floor > 0");
@@ -2583,10 +2671,11 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
     if (!a->k_cache || !a->v_cache || a->num_blocks <= 0 || a->block_size <= 0)
       return fail(SLO_ERR_INVALID, "paged_attention: the KV write needs the pool");
     const int64_t row = (int64_t)a->num_kv_heads * HD;
-    // Launches without prefill rows address each new row by its own stride, so
-    // views of a fused projection's output fold as well (prefill tiles of new
-    // tokens take the pool's row length).
-    const bool strided = (a->phases & SLO_NEW_ROWS_STRIDED) && !do_pf;
+    // Launches that read no new row through a table beside pool rows (no
+    // prefill rows, or only cold ones) address each new row by its own stride,
+    // so views of a fused projection's output fold as well (prefill tiles of
+    // new tokens take the pool's row length).
+    const bool strided = (a->phases & SLO_NEW_ROWS_STRIDED) && (!do_pf || cold);
     auto bad_stride = [&](int64_t st) { return strided ? st < row || st % 8 : st != row; };
     if (!a->new_k || !a->new_v || a->num_new_rows != a->num_q_rows || bad_stride(a->new_k_row_stride) ||
         bad_stride(a->new_v_row_stride) || (reinterpret_cast<uintptr_t>(a->new_k) % 16) ||
@@ -2594,7 +2683,7 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
       return fail(SLO_ERR_INVALID,
                   "paged_attention: new K/V must be contiguous 16-byte aligned bf16 rows, one per query row");
   }
-  if (store && !fold) {
+  if (store && !fold && !cold) {
     const int rc = slo_store_kvcache(a->new_k, a->new_k_row_stride, a->new_v, a->new_v_row_stride,
                                      a->store_slot_mapping, a->num_new_rows, a->num_kv_heads, HD, a->kv_dtype,
                                      const_cast<void*>(a->k_cache), const_cast<void*>(a->v_cache),
@@ -2671,12 +2760,13 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
   p.counters = reinterpret_cast<int*>(wsb + CTRL_BYTES);
   p.partials = reinterpret_cast<float*>(wsb + PARTIALS_OFFSET);
   p.pf_split_bytes = pf_split_bytes;
-  p.sslots = fold ? a->store_slot_mapping : nullptr;
+  p.sslots = fold || cold ? a->store_slot_mapping : nullptr;
   p.nk = static_cast<const uint16_t*>(a->new_k);
   p.nv = static_cast<const uint16_t*>(a->new_v);
   p.nk_stride = a->new_k_row_stride;
   p.nv_stride = a->new_v_row_stride;
-  p.nnew = fold ? a->num_new_rows : 0;
+  p.nnew = fold || cold ? a->num_new_rows : 0;
+  p.store_fp8 = fp8 ? 1 : 0;
   p.scale_floor = a->store_scale_floor;
   p.num_slots = (int64_t)a->num_blocks * a->block_size;
   // A merge task waits up to 200 ms for its chunks (a whole decode launch
@@ -2700,7 +2790,7 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
   // cold prefill rows (new K/V only) runs the bf16 one, which holds fewer
   // registers.
   const bool fp8_reads = fp8 && (do_dec || (do_pf && p.ptab != nullptr));
-  const int mode = do_dec && do_pf ? MODE_MIXED : do_pf ? MODE_PREFILL : MODE_DECODE;
+  const int mode = do_dec && do_pf ? MODE_MIXED : !do_pf ? MODE_DECODE : p.ptab ? MODE_PREFILL : MODE_COLD;
   // With the KV write folded in, the pool's format decides the instantiation
   // (its store quantises); otherwise what the launch reads does.
   const bool kfp8 = fold ? fp8 : fp8_reads;

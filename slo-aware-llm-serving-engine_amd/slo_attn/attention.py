@@ -58,10 +58,13 @@ class Attention(nn.Module):
         # launch less) in decode steps, also from views of the QKV projection
         # and into E4M3FN pools (at most 8 query heads per kv head): 16 rows of
         # 64-1,024 tokens 18.1 -> 16.8 us a layer, 64 rows of 512-4,096 125.6
-        # -> 124.2 us, 40 E4M3FN rows of 256-4,096 51.3 -> 49.2 us.  A prefill step folds contiguous bf16 rows; otherwise
-        # the store kernel runs first.
+        # -> 124.2 us, 40 E4M3FN rows of 256-4,096 51.3 -> 49.2 us.  So do cold
+        # prefill steps (no block tables), whose items write their own tokens.
+        # A prefill step that reads the pool hands over contiguous bf16 rows
+        # only; otherwise the store kernel runs first.
+        paged = context.is_prefill and context.block_tables is not None
         fold = have_cache and not kv_stored and (
-            self.k_scale is None and foldable(k, v) if context.is_prefill
+            self.k_scale is None and foldable(k, v) if paged
             else foldable_strided(k, v) and (self.k_scale is None or q.shape[1] <= 8 * k.shape[1]))
         if fold:
             check_store(k, v, k_cache, v_cache, context.slot_mapping, *self._scales())
@@ -70,15 +73,15 @@ class Attention(nn.Module):
         store = dict(store_slot_mapping=context.slot_mapping, new_k=k, new_v=v) if fold else {}
         if context.is_prefill:
             rows = context.cu_seqlens_q.numel() - 1
-            paged = context.block_tables is not None
             pool = paged or fold
             return paged_attention(
                 q, k_cache if pool else None, v_cache if pool else None, self.scale,
-                num_kv_heads=self.num_kv_heads, k_scale=self.k_scale if paged else None,
-                v_scale=self.v_scale if paged else None, num_prefill=rows,
+                num_kv_heads=self.num_kv_heads, k_scale=self.k_scale if pool else None,
+                v_scale=self.v_scale if pool else None, num_prefill=rows,
                 prefill_cu_q=context.cu_seqlens_q, prefill_cu_k=context.cu_seqlens_k,
                 max_q=context.max_seqlen_q, max_k=context.max_seqlen_k,
-                prefill_tables=context.block_tables, k=None if paged else k, v=None if paged else v, **store)
+                prefill_tables=context.block_tables, k=None if paged else k, v=None if paged else v,
+                phases=_lib.PHASE_ALL if paged else _lib.PHASE_ALL | _lib.NEW_ROWS_STRIDED, **store)
         o = paged_attention(
             q, k_cache, v_cache, self.scale, num_kv_heads=self.num_kv_heads,
             k_scale=self.k_scale, v_scale=self.v_scale, num_decode=q.shape[0],

@@ -57,12 +57,13 @@ def forward_mixed(q, k, v, k_cache, v_cache, context, scale, store_fn,
     # decode rows and two chunks, one after a 1,024-token prefix: 108 against
     # 72 us), and cold rows run in the E4M3FN instantiation, which spills
     # registers (4 cold rows: 134 against 107 us).
-    # Pure decode steps also fold rows that are views of the QKV projection.
-    decode_only = not meta.num_prefill_tokens
+    # Pure decode steps, and steps of cold prefill rows only (they read no
+    # pool), also fold rows that are views of the QKV projection.
+    alone = not meta.num_prefill_tokens or (not meta.num_decode and not meta.prefill_has_history)
     fold = (store_fn is store_kvcache and phases == _lib.PHASE_ALL
-            and (foldable_strided(k, v) if decode_only else foldable(k, v))
-            and (k_scale is None or (q.shape[1] <= 8 * k.shape[1] and decode_only)))
-    if fold and decode_only:
+            and (foldable_strided(k, v) if alone else foldable(k, v))
+            and (k_scale is None or (q.shape[1] <= 8 * k.shape[1] and alone)))
+    if fold and alone:
         phases |= _lib.NEW_ROWS_STRIDED
     if fold:
         check_store(k, v, k_cache, v_cache, context.slot_mapping, k_scale, v_scale)

@@ -362,3 +362,55 @@ def test_decode_folds_views_of_the_qkv_projection(device, fp8, rows, hi, hkv):
                             k_scale=got_pools[2] if fp8 else None, v_scale=got_pools[3] if fp8 else None,
                             num_decode=rows, decode_lens=dl, decode_tables=padded, store_slot_mapping=slots,
                             new_k=k, new_v=v)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens,hq,hkv", [([1], 32, 8), ([31, 33, 1, 64, 100], 8, 8), ([700, 257], 64, 8),
+                                         ([1813, 346, 16], 32, 8)])
+def test_cold_prefill_items_write_the_new_rows(device, fp8, lens, hq, hkv):
+    # A launch of cold prefill rows reads no pool: its items write their own
+    # blocks' tokens (all kv heads, head groups once), and new rows outside
+    # every prefill row follow (here three padding tokens, one with a slot).
+    # Views of the QKV projection and contiguous rows, through
+    # Attention.forward's V0 branch and forward_mixed, against the store kernel
+    # followed by the launch: outputs and pool bytes.
+    g = torch.Generator().manual_seed(sum(lens) + hq)
+    dh, bs, n = 128, 256, sum(lens)
+    total, nblk = n + 3, (n + 3 + 255) // 256 + 2
+    slot = torch.randperm(nblk * bs, generator=g)[:total].to(torch.int32)
+    slot[n], slot[n + 2], slot[0] = -1, nblk * bs, -1  # skipped: -1 and past the pool
+    slots = slot.to(device)
+    qkv = torch.randn(total, (hq + 2 * hkv) * dh, generator=g).to(torch.bfloat16).to(device)
+    q, k, v = (t.view(total, -1, dh) for t in qkv.split([hq * dh, hkv * dh, hkv * dh], -1))
+    q = q.contiguous()
+    cu = [0]
+    for x in lens:
+        cu.append(cu[-1] + x)
+    cu = torch.tensor(cu, dtype=torch.int32, device=device)
+    reserve_workspace(device, 0, 0, hq, hkv, dh)
+
+    def pools():
+        if not fp8:
+            return [torch.full((nblk, bs, hkv, dh), x, dtype=torch.bfloat16, device=device) for x in (3.0, -3.0)]
+        return ([torch.full((nblk, bs, hkv, dh), 7, dtype=torch.uint8, device=device) for _ in range(2)]
+                + [torch.full((nblk, bs, hkv), 9.0, device=device) for _ in range(2)])
+
+    meta = MixedAttentionContext(0, total, None, None, cu, cu, None, max(lens), max(lens), False)
+    ctx = SimpleNamespace(mixed=meta, slot_mapping=slots)
+    for kk, vv in ((k, v), (k.contiguous(), v.contiguous())):
+        a, b, c = pools(), pools(), pools()
+        ref = forward_mixed(q, kk, vv, a[0], a[1], ctx, dh ** -0.5, _two_launch_store, *a[2:])
+        got = forward_mixed(q, kk, vv, b[0], b[1], ctx, dh ** -0.5, store_kvcache, *b[2:])
+        attn = Attention(hq, dh, dh ** -0.5, hkv)
+        attn.k_cache, attn.v_cache = c[:2]
+        if fp8:
+            attn.k_scale, attn.v_scale = c[2:]
+        set_context(True, cu, cu, max(lens), max(lens), slots)
+        v0 = attn(q, kk, vv)
+        reset_context()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+        assert torch.equal(v0.view(torch.int16), ref.view(torch.int16))
+        for x, y, z in zip(a, b, c):
+            assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
+            assert torch.equal(x.view(torch.uint8), z.view(torch.uint8))
