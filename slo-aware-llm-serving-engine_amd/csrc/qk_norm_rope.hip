@@ -21,9 +21,15 @@
 // One 512-thread workgroup per token; a 16-lane group per head of the QKV
 // row, lane j holding elements 8j..8j+7 (one 16-byte load), so a head's
 // statistics are a 16-lane reduction and the RoPE partner of element d
-// (d +- 64) sits in lane j ^ 8.  (256-thread workgroups, three heads per
-// group at Qwen3-4B's 48 heads, took 10.0 instead of 9.4 us for 1,048
-// tokens; one head per group, 768 threads, 9.6 us.)
+// (d +- 64) sits in lane j ^ 8.  Bound by VALU issue at many tokens (28.5 MB
+// for 1,048 tokens are 5.6 us of a copy) and by one dependent chain of loads
+// at few: the sums reduce by DPP moves instead of LDS permutes, the fp64
+// square root and division are one refined v_rsq_f64, the sine is negated
+// once per token instead of choosing between two results per element, and
+// rows are addressed by a uniform base and a 32-bit offset: 9.6 -> 8.5 us for
+// 1,048 tokens, graph-replayed.  (384 threads, two heads in every group:
+// 9.1 us; 256 threads and three heads, before these changes, 10.0 against
+// 9.4 us; one head per group, 768 threads, 9.6 us.)
 #include "common.h"
 #include "capi_internal.h"
 
@@ -32,6 +38,41 @@ namespace slo {
 constexpr int QK_HD = 128;
 constexpr int QK_NT = 512;   // threads per workgroup: 32 groups of 16 lanes
 constexpr int QK_UNITS = 2;  // heads per 16-lane group: rows of up to 64 heads
+
+// 16 bytes at a uniform base plus a 32-bit lane offset in bytes (the base stays
+// in SGPRs; every head offset of a row is below 2^14).
+__device__ __forceinline__ void st16_at(uint16_t* base, int off, const u32x4& v) {
+  *reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(base) + (uint32_t)off) = v;
+}
+
+// x plus the lane that DPP control CTRL names in the row of 16.
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xf, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+  return x + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// Sum over the 16 lanes of a row, the same bits in every lane: neighbours,
+// then pairs, then the mirrored quad and the mirrored half (each already
+// uniform), by DPP moves.
+__device__ __forceinline__ double row_sum(double x) {
+  x = add_dpp<0xb1>(x);    // quad_perm 1, 0, 3, 2
+  x = add_dpp<0x4e>(x);    // quad_perm 2, 3, 0, 1
+  x = add_dpp<0x141>(x);   // row_half_mirror
+  return add_dpp<0x140>(x);  // row_mirror
+}
+// 1 / sqrt(x) rounded to fp32 from an fp64 value within about an ulp:
+// v_rsq_f64's 2^-23 refined once (third order) instead of the library's fp64
+// square root and division (about 50 instructions).  0, inf and NaN keep
+// v_rsq_f64's own result.
+__device__ __forceinline__ float rsqrt_rounded(float v) {
+  const double x = (double)v;
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * y, y, 1.0);
+  const double r = __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+  return (float)(e == e ? r : y);
+}
 
 // One (token, head) unit: lane j of the 16-lane group holds elements 8j..8j+7
 // of head hh in x.  Writes q_out, or k_out and the pool, or the pool.
@@ -56,11 +97,9 @@ __device__ __forceinline__ void qk_unit(const u32x4& x, int hh, int j, int64_t t
     // mean is rounded to fp32 once whatever the summation order.
     double ss = 0.0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) ss += (double)f[i] * (double)f[i];
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m, 64);
-    const float var = (float)(ss / QK_HD);
-    const float r = (float)(1.0 / sqrt((double)(var + eps)));
+    for (int i = 0; i < 8; ++i) ss = __builtin_fma((double)f[i], (double)f[i], ss);
+    const float var = (float)(row_sum(ss) * (1.0 / QK_HD));
+    const float r = rsqrt_rounded(var + eps);
     const u32x4 wv = is_q ? wq : wk;
     // bf16 roundings by v_cvt_pk_bf16_f32 (round to nearest even), two values each.
     float n[8];
@@ -77,17 +116,16 @@ __device__ __forceinline__ void qk_unit(const u32x4& x, int hh, int j, int64_t t
     for (int i = 0; i < 8; ++i) {
       // element d +- 64: lane j ^ 8 of the 16-lane row (DPP row rotate by 8)
       const float other = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(n[i]), 0x128, 0xf, 0xf, false));
-      const float a = n[i] * c[i], b = other * s[i];
-      y[i] = j < 8 ? a - b : a + b;  // lanes 0-7: x1 half, lanes 8-15: x2 half
+      y[i] = n[i] * c[i] + other * s[i];  // s is negated in lanes 0-7 (x1 half)
     }
     u32x4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(y[2 * i], y[2 * i + 1]);
     if (is_q) {
-      *reinterpret_cast<u32x4*>(q_out + (tok * num_heads + hh) * QK_HD + d0) = o;
+      st16_at(q_out + tok * num_heads * QK_HD, 2 * (hh * QK_HD + d0), o);
       return;
     }
-    *reinterpret_cast<u32x4*>(k_out + (tok * num_kv_heads + kvh) * QK_HD + d0) = o;
+    st16_at(k_out + tok * num_kv_heads * QK_HD, 2 * (kvh * QK_HD + d0), o);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       f[2 * i] = __uint_as_float(o[i] << 16);
@@ -96,16 +134,17 @@ __device__ __forceinline__ void qk_unit(const u32x4& x, int hh, int j, int64_t t
   }
   if (!store) return;
   // K (normalised and rotated) or V (as given) into the pool.
-  const int64_t dst = (slot * num_kv_heads + kvh) * QK_HD + d0;
+  const int64_t row0 = slot * num_kv_heads * QK_HD;  // the token's first element in the pool
+  const int off = kvh * QK_HD + d0;
   if (kv_dtype == KV_BF16) {
     u32x4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = (__float_as_uint(f[2 * i]) >> 16) | (__float_as_uint(f[2 * i + 1]) & 0xffff0000u);
-    *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(is_k ? k_cache : v_cache) + dst) = o;
+    st16_at(static_cast<uint16_t*>(is_k ? k_cache : v_cache) + row0, 2 * off, o);
   } else {
     float scale;
     const u32x2 codes = e4m3_encode8<16>(f, scale_floor, scale);
-    *reinterpret_cast<u32x2*>(static_cast<uint8_t*>(is_k ? k_cache : v_cache) + dst) = codes;
+    *reinterpret_cast<u32x2*>(static_cast<uint8_t*>(is_k ? k_cache : v_cache) + row0 + off) = codes;
     if (j == 0) (is_k ? k_scale : v_scale)[slot * num_kv_heads + kvh] = scale;
   }
 }
@@ -128,12 +167,12 @@ qk_norm_rope_store_kernel(const uint16_t* __restrict__ qkv, int64_t qkv_stride, 
   // dependent load), then the row's heads and the norm weights.
   int64_t pos = positions[tok];
   const int64_t slot = slot_mapping[tok];
-  const uint16_t* row = qkv + tok * qkv_stride + 8 * j;
+  const uint8_t* row = reinterpret_cast<const uint8_t*>(qkv + tok * qkv_stride);
   u32x4 x[QK_UNITS];
 #pragma unroll
   for (int it = 0; it < QK_UNITS; ++it) {
     const int hh = grp + (QK_NT / 16) * it;
-    x[it] = hh < heads ? *reinterpret_cast<const u32x4*>(row + (int64_t)hh * QK_HD) : u32x4{0, 0, 0, 0};
+    x[it] = hh < heads ? *reinterpret_cast<const u32x4*>(row + (uint32_t)(2 * (hh * QK_HD + 8 * j))) : u32x4{0, 0, 0, 0};
   }
   const u32x4 wq = *reinterpret_cast<const u32x4*>(q_w + 8 * j);
   const u32x4 wk = *reinterpret_cast<const u32x4*>(k_w + 8 * j);
@@ -142,7 +181,12 @@ qk_norm_rope_store_kernel(const uint16_t* __restrict__ qkv, int64_t qkv_stride, 
   const f32x4 c0 = *reinterpret_cast<const f32x4*>(cs), c1 = *reinterpret_cast<const f32x4*>(cs + 4);
   const f32x4 s0 = *reinterpret_cast<const f32x4*>(cs + 64), s1 = *reinterpret_cast<const f32x4*>(cs + 68);
   const float c[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
-  const float s[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+  // Lanes 0-7 hold the x1 half: x1 * cos - x2 * sin, the same bits as adding
+  // x2 times the negated sine.
+  const uint32_t neg = j < 8 ? 0x80000000u : 0u;
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s[i] = __uint_as_float(__float_as_uint(i < 4 ? s0[i] : s1[i - 4]) ^ neg);
   const bool store = slot >= 0 && slot < num_slots;
 #pragma unroll
   for (int it = 0; it < QK_UNITS; ++it) {

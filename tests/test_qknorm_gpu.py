@@ -171,3 +171,22 @@ def test_mixed_step_with_fused_write_equals_separate_write(device, fp8):
 def _ctx(slot_t, meta):
     from slo_attn.context import Context
     return Context(is_prefill=False, slot_mapping=slot_t, mixed=meta)
+
+
+def test_statistics_over_the_exponent_range_bit_exact(device):
+    # The reciprocal square root is one refined v_rsq_f64: token t scales its
+    # row by 2^(4t - 80), from sums that vanish beside eps to means past fp32
+    # (inf: the row becomes zeros, as 1 / sqrt(inf) does in the oracle), and
+    # one row is zero throughout.
+    n, hq, hkv = 46, 8, 2
+    _, qkv, pos, slots, qw, kw, kc, vc, _, _ = _case(n, hq, hkv, 1, False, seed=21)
+    qkv = (qkv.float() * torch.exp2(4.0 * torch.arange(n) - 80)[:, None]).to(torch.bfloat16)
+    qkv[7] = 0
+    table = rope_cos_sin(HD, 40960, 1e6, "cpu")
+    q, k, _ = qk_norm_rope_store(qkv.to(device), pos.to(device), qw.to(device), kw.to(device), EPS, table.to(device),
+                                 hq, hkv, kc.to(device), vc.to(device), slots.to(device))
+    with np.errstate(over="ignore", divide="ignore"):
+        qo, ko, _ = qknorm.qkv_step_store(_bits(qkv), pos.numpy(), _bits(qw), _bits(kw), EPS, table.numpy(), hq, hkv,
+                                          slots.numpy(), _bits(kc).copy(), _bits(vc).copy(), None, None)
+    assert torch.isfinite(qkv.float()).all()
+    assert np.array_equal(_bits(q), qo) and np.array_equal(_bits(k), ko)
