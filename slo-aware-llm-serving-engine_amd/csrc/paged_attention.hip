@@ -2526,7 +2526,10 @@ DirectKernel direct_kernel(bool fold, bool fp8) {
 // run the work lists.  Measured on rows of 64-8192 tokens: the direct kernel
 // wins up to these sizes (16 rows of 64-1024 tokens 30 -> 15 us, 24 rows of
 // 256-4096 53 -> 51 us bf16 and 41 -> 37 us E4M3FN), the work lists beyond.
-constexpr int DIRECT_MAX_ROUNDS[2] = {4, 2};
+// (E4M3FN, table width 4,096 tokens: 40 rows of 256-4,096, a grid of 2.5 times,
+// 56.0 -> 51.0 us; 48 rows of 512-4,096, 3 times, 61.4 -> 57.9; 64 rows, 4
+// times, 71.2 with the work lists against 76.0.)
+constexpr int DIRECT_MAX_ROUNDS[2] = {4, 3};
 constexpr int DIRECT_CHUNK_MAX = 1024;  // tokens
 
 // Compute units and, per instantiation, the workgroups one CU holds at once
