@@ -103,6 +103,11 @@ __device__ __forceinline__ void dma16_at(const void* base, uint32_t off, uint32_
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
                : "memory", "m0");
 }
+// With the non-temporal policy (see dma16_nt).
+__device__ __forceinline__ void dma16_nt_at(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
 // Four LDS-DMA loads that fill 4 KiB of LDS from one M0 write: load i lands
 // at lds + 1024 i and reads base + o[i] + 1024 i (the instruction offset is
 // added to the global and the LDS address alike), so the caller passes o[i]

@@ -38,7 +38,12 @@ def _check_tokens(tokens, ref_logits_bits):
     return (tokens == np.argmax(lf, axis=1)).mean()
 
 
-@pytest.mark.parametrize("rows,vocab,hidden", [(1, 1000, 128), (7, 5003, 512), (65, 3000, 2560), (128, 777, 256)])
+# Up to 64 rows the weight streams through LDS in 128-row blocks of 128-column
+# chunks (one chunk per row, a ragged last block, more blocks than workgroups);
+# 8 KiB weight rows keep the register kernel up to 32 rows.
+@pytest.mark.parametrize("rows,vocab,hidden", [(1, 1000, 128), (7, 5003, 512), (65, 3000, 2560), (128, 777, 256),
+                                               (16, 129, 256), (17, 70001, 128), (33, 34000, 384), (64, 127, 640),
+                                               (32, 300, 4096), (40, 300, 4096)])
 def test_against_oracle(device, rows, vocab, hidden):
     g = torch.Generator().manual_seed(rows + vocab)
     h = torch.randn(rows, hidden, generator=g).to(torch.bfloat16)
