@@ -46,17 +46,16 @@ def forward_mixed(q, k, v, k_cache, v_cache, context, scale, store_fn,
         raise RuntimeError("mixed forward requires an allocated KV pool")
     # The library's own store runs inside the attention launch when the new
     # rows are contiguous and the step has decode rows (same result, one
-    # launch less; a step without decode rows gets the store kernel first from
-    # the same call, so that its long rows can split their keys over
-    # 32-position blocks); any other store_fn runs first.  An E4M3FN pool folds it into pure decode steps only (with at
-    # most 8 query heads per kv head): the launch then quantises each decode
-    # row's newest token itself (16 rows of 64-1,024 tokens: 25.3 us, against
-    # the store kernel and a 24.1 us launch).  With prefill rows the folded
-    # E4M3FN launch measured slower than the store kernel and the launch: rows
-    # reading the pool re-quantise their new tokens' tiles in every item (24
-    # decode rows and two chunks, one after a 1,024-token prefix: 108 against
-    # 72 us), and cold rows run in the E4M3FN instantiation, which spills
-    # registers (4 cold rows: 134 against 107 us).
+    # launch less; a step of prefill rows that read the pool gets the store
+    # kernel first from the same call, so that its long rows can split their
+    # keys over 32-position blocks); any other store_fn runs first.  An E4M3FN
+    # pool folds it only into pure decode steps (with at most 8 query heads per
+    # kv head: the launch quantises each decode row's newest token itself) and
+    # steps of cold prefill rows, whose items quantise their own tokens.  With
+    # decode and prefill rows the folded E4M3FN launch measured slower than the
+    # store kernel and the launch: rows reading the pool re-quantise their new
+    # tokens' tiles in every item (24 decode rows and two chunks, one after a
+    # 1,024-token prefix: 108 against 72 us).
     # Pure decode steps, and steps of cold prefill rows only (they read no
     # pool), also fold rows that are views of the QKV projection.
     alone = not meta.num_prefill_tokens or (not meta.num_decode and not meta.prefill_has_history)
