@@ -21,6 +21,7 @@ exact_history=True)``).
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -40,15 +41,21 @@ class MixedStepBuffers:
         self.width, self.block_size, self.max_model_len = table_width, block_size, max_model_len
         self.device = torch.device(device)
         rows = decode_capacity + prefill_capacity
-        # one host-to-device copy per step: [row_start | row_tokens | tables | input ids]
-        self._host = torch.zeros(2 * rows + rows * table_width + token_capacity, dtype=torch.int64,
-                                 pin_memory=True)
+        # One host-to-device copy per step, in the types the kernels read: token
+        # ids (int64), then row starts, row token counts and block tables
+        # (int32).  The buffers below are views of it, so no conversion kernels
+        # run before the captured step.
+        words = 2 * rows + rows * table_width
+        self._host = torch.zeros(8 * token_capacity + 4 * words, dtype=torch.uint8, pin_memory=True)
         self._packed = torch.zeros_like(self._host, device=self.device)
-        p = self._packed
-        self.row_start32 = torch.zeros(rows, dtype=torch.int32, device=self.device)
-        self.row_tokens32 = torch.zeros(rows, dtype=torch.int32, device=self.device)
-        self.tables = torch.full((rows, table_width), -1, dtype=torch.int32, device=self.device)
-        self.input_ids = p[2 * rows + rows * table_width:]
+        self.input_ids = self._packed[:8 * token_capacity].view(torch.int64)
+        p = self._packed[8 * token_capacity:].view(torch.int32)
+        self.row_start32, self.row_tokens32 = p[:rows], p[rows:2 * rows]
+        self.tables = p[2 * rows:].view(rows, table_width)
+        self.tables.fill_(-1)
+        h = self._host.numpy()
+        self._ids = h[:8 * token_capacity].view(np.int64)
+        self._words = h[8 * token_capacity:].view(np.int32)
         self.positions = torch.zeros(token_capacity, dtype=torch.int64, device=self.device)
         self.slot_mapping = torch.full((token_capacity,), -1, dtype=torch.int32, device=self.device)
         self.decode_lens = torch.zeros(max(decode_capacity, 1), dtype=torch.int32, device=self.device)
@@ -67,28 +74,22 @@ class MixedStepBuffers:
         if len(tables) != d + r or any(len(t) > self.width for t in tables):
             raise ValueError("one block table per row, at most table_width entries")
         rows = self.dc + self.pc
-        h = self._host
+        ids, h = self._ids, self._words
         self._copied.synchronize()  # the previous step's copy has left the pinned buffer
-        h.zero_()
-        start, tok = h[:rows], h[rows:2 * rows]
-        tab = h[2 * rows:2 * rows + rows * self.width].view(rows, self.width)
-        tab.fill_(-1)
-        ids = h[2 * rows + rows * self.width:]
-        for b, s in enumerate(decode_start):
-            start[b], tok[b] = s, 1
-            tab[b, :len(tables[b])] = torch.tensor(tables[b], dtype=torch.int64)
-            ids[b] = input_ids[b]
-        at = d
+        ids[:] = 0
+        h[:2 * rows] = 0
+        h[2 * rows:] = -1
+        start, tok, tab = h[:rows], h[rows:2 * rows], h[2 * rows:].reshape(rows, self.width)
+        start[:d] = decode_start
+        tok[:d] = 1
         for i, (s, n) in enumerate(prefill_rows):
             start[self.dc + i], tok[self.dc + i] = s, n
-            tab[self.dc + i, :len(tables[d + i])] = torch.tensor(tables[d + i], dtype=torch.int64)
-        ids[self.dc:self.dc + len(input_ids) - d] = torch.tensor(input_ids[d:], dtype=torch.int64)
-        self._packed.copy_(h, non_blocking=True)
+        for i, t in enumerate(tables):
+            tab[i if i < d else self.dc + i - d, :len(t)] = t
+        ids[:d] = input_ids[:d]
+        ids[self.dc:self.dc + len(input_ids) - d] = input_ids[d:]
+        self._packed.copy_(self._host, non_blocking=True)
         self._copied.record()
-        p = self._packed
-        self.row_start32.copy_(p[:rows])
-        self.row_tokens32.copy_(p[rows:2 * rows])
-        self.tables.copy_(p[2 * rows:2 * rows + rows * self.width].view(rows, self.width))
 
     def build(self) -> None:
         """Derives the step's metadata on the GPU (capturable)."""
