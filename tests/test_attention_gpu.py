@@ -301,3 +301,59 @@ def test_prefill_exponent_offsets_move(device, kv_fp8, rising):
         case.v = (case.v.float() / 4).to(torch.bfloat16)
         case.old_v = [(v.float() / 4).to(torch.bfloat16) for v in case.old_v]
         _check(case, device)
+
+
+@pytest.mark.parametrize("n", [64, 100])
+def test_prefill_dominating_key_is_exact(device, n):
+    # A key whose probability exceeds 2^8 times the offset's moves the offset,
+    # so its own probability is exactly 1 and not a value above 2^8 rounded to
+    # bf16.  Key 40 (second half tile; the first one leaves the offset at score
+    # 0) has probabilities of 257 to 330 over kv heads and queries, all other
+    # keys 1 and every V 1: the outputs are 1, and a rounding of the dominating
+    # probability by more than 0.2% of the sum shows (bf16 steps below 1 are
+    # 2^-8, halves of them 0.195%).  After the move the other keys' common
+    # rounding is at most n * 2^-8 * 2^-9 of the sum: below 0.08%.
+    from slo_attn import paged_attention
+    hkv, dh = 8, 128
+    scale = dh ** -0.5
+    a = torch.arange(7.875, 8.5, 0.03125).to(torch.bfloat16).unique()
+    q = torch.zeros(n, 4 * hkv, dh)
+    q[:, :, 0] = a.float()[torch.arange(n) % len(a)][:, None]
+    k = torch.zeros(n, hkv, dh)
+    k[40, :, 0] = (8.0 + 0.0625 * torch.arange(hkv)).to(torch.bfloat16).float()
+    p = torch.exp2(q[41:, :, 0] * k[40, :, 0].repeat_interleave(4)[None] * scale * 1.4426950408889634)
+    rows = (p > 257) & (p < 330)
+    off = 1.0 + (p.to(torch.bfloat16).float() - p) / (p + torch.arange(41, n)[:, None])
+    assert (rows & (off < 0.998)).sum() > 10  # what an offset left alone would return
+    cu = torch.tensor([0, n], dtype=torch.int32, device=device)
+    to = lambda x: x.to(torch.bfloat16).to(device)  # noqa: E731
+    out = paged_attention(to(q), None, None, scale, num_kv_heads=hkv, num_prefill=1, prefill_cu_q=cu, prefill_cu_k=cu,
+                          max_q=n, max_k=n, k=to(k), v=torch.ones(n, hkv, dh, dtype=torch.bfloat16, device=device))
+    assert torch.equal(out[41:].float().cpu()[rows], torch.ones(int(rows.sum()), dh))
+
+
+@pytest.mark.parametrize("decode", [[], [40]])
+@pytest.mark.parametrize("hist,count", [([0], [200]), ([0, 300], [97, 130]), ([1500], [64])])
+def test_prefill_infinities_and_nan(device, decode, hist, count):
+    # A NaN key makes every query that sees it NaN in its kv head; an infinite
+    # one gives scores of +inf (NaN outputs) or -inf (probability 0) by the sign
+    # of the query's element; every other output stays within the gate.
+    case = Case(decode, hist, count, hq=8, hkv=2, seed=31)
+    case.k[-50, 0, 3] = float("nan")
+    case.k[-40, 1, 5] = float("inf")
+    want, at = [], 0
+    for old_k, old_v, m in zip(case.old_k, case.old_v, [1] * len(decode) + count):
+        q = case.q[at:at + m].float()
+        k, v = (torch.cat((old, new[at:at + m])).float().repeat_interleave(4, 1)
+                for old, new in ((old_k, case.k), (old_v, case.v)))
+        s = (q[:, :, None] * k.transpose(0, 1)[None]).sum(-1) * case.scale  # [m, heads, keys]
+        s.masked_fill_(torch.arange(k.shape[0]) > torch.arange(m)[:, None, None] + old_k.shape[0], float("-inf"))
+        p = s.softmax(-1)
+        want.append((p[..., None] * v.transpose(0, 1)[None]).sum(2))
+        at += m
+    want = torch.cat(want)
+    got, _ = case.run_gpu(device)
+    got = got.float().cpu()
+    seen = torch.isnan(want)
+    assert seen.any() and not seen.all() and torch.equal(torch.isnan(got), seen)
+    assert_close_gate(torch.where(seen, 0.0, got), torch.where(seen, 0.0, want))
