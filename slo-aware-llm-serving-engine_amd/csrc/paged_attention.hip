@@ -1438,14 +1438,15 @@ __global__ void __launch_bounds__(NT, 2) decode_direct_kernel(Params p, int nch_
 
   // Once per workgroup, on every path (after the item's loads are issued
   // where it has one): its share of the KV write (4 * NT pieces per
-  // workgroup) and of the zeros for query rows past every decode and prefill
-  // row.
+  // workgroup and turn: a launch may have many more query rows, each with a
+  // new row, than decode rows) and of the zeros for query rows past every
+  // decode and prefill row.
   auto side_work = [&]() {
     bool any = false;
     if constexpr (FOLD) {
       const int64_t per_wg = 4 * NT, all = (int64_t)p.nnew * (2 * (p.hkv * HD / 8));
-      if ((int64_t)x * per_wg < all) {
-        store_new_rows<FP8>(p, (int64_t)x * per_wg, min(all, (int64_t)(x + 1) * per_wg), tid);
+      for (int64_t i = (int64_t)x * per_wg; i < all; i += (int64_t)gridDim.x * per_wg) {
+        store_new_rows<FP8>(p, i, min(all, i + per_wg), tid);
         any = true;
       }
     }

@@ -414,3 +414,36 @@ def test_cold_prefill_items_write_the_new_rows(device, fp8, lens, hq, hkv):
         for x, y, z in zip(a, b, c):
             assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
             assert torch.equal(x.view(torch.uint8), z.view(torch.uint8))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("strided", [False, True])
+def test_decode_launch_stores_every_new_row(device, fp8, strided):
+    # One decode row and 900 query rows, all with a slot: the launch's small
+    # grid (64 workgroups) takes the new rows in several turns.  Pool bytes of
+    # the store kernel, and zeros in the output rows past the decode row.
+    g = torch.Generator().manual_seed(3)
+    rows, hq, hkv, dh, bs, nblk = 900, 32, 8, 128, 256, 6
+    slots = torch.randperm((nblk - 1) * bs, generator=g)[:rows].to(torch.int32)
+    slots[0] = (nblk - 1) * bs + 69
+    slots, dl = slots.to(device), torch.tensor([70], dtype=torch.int32, device=device)
+    table = torch.tensor([[nblk - 1]], dtype=torch.int32, device=device)
+    qkv = torch.randn(rows, (hq + 2 * hkv) * dh, generator=g).to(torch.bfloat16).to(device)
+    q, k, v = (t.view(rows, -1, dh) for t in qkv.split([hq * dh, hkv * dh, hkv * dh], -1))
+    q = q.contiguous()
+    if not strided:
+        k, v = k.contiguous(), v.contiguous()
+    ctx = SimpleNamespace(mixed=MixedAttentionContext(1, 0, dl, table, None, None, None, 0, 0), slot_mapping=slots)
+    outs, pools = [], []
+    for store in (_two_launch_store, store_kvcache):
+        if fp8:
+            pool = [torch.full((nblk, bs, hkv, dh), 7, dtype=torch.uint8, device=device) for _ in range(2)]
+            pool += [torch.full((nblk, bs, hkv), 9.0, device=device) for _ in range(2)]
+        else:
+            pool = [torch.full((nblk, bs, hkv, dh), x, dtype=torch.bfloat16, device=device) for x in (3.0, -3.0)]
+        outs.append(forward_mixed(q, k, v, pool[0], pool[1], ctx, dh ** -0.5, store, *pool[2:]))
+        pools.append(pool)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16)) and not outs[1][1:].any()
+    for a, b in zip(*pools):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
