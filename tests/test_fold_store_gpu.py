@@ -447,3 +447,41 @@ def test_decode_launch_stores_every_new_row(device, fp8, strided):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16)) and not outs[1][1:].any()
     for a, b in zip(*pools):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("head,length,rows", [(0, 40, 1500), (70, 33, 200), (31, 1, 65), (33, 0, 40)])
+def test_cold_launch_writes_rows_outside_every_prefill_row(device, fp8, head, length, rows):
+    # A cold prefill row at [head, head + length) of `rows` new rows: the rows
+    # before and after it are written in blocks of 32, at the edges of a block
+    # and with blocks whose slots are all -1 or past the pool, in part or not
+    # at all.  Pool bytes of the store kernel; the attention output is that of
+    # the launch without the write.
+    g = torch.Generator().manual_seed(head + rows)
+    hq, hkv, dh, bs, nblk = 16, 4, 128, 256, 7
+    slot = torch.randperm(nblk * bs, generator=g)[:rows].to(torch.int32)
+    slot[head + length:head + length + 32] = -1
+    slot[-40:-1] = -1
+    slot[head // 2:head // 2 + 3] = nblk * bs
+    slots = slot.to(device)
+    q = torch.randn(rows, hq, dh, generator=g).to(torch.bfloat16).to(device)
+    k, v = (torch.randn(rows, hkv, dh, generator=g).to(torch.bfloat16).to(device) for _ in range(2))
+    cu = torch.tensor([head, head + length], dtype=torch.int32, device=device)
+    reserve_workspace(device, 0, 0, hq, hkv, dh)
+    a, b = [], []
+    for pool in (a, b):
+        if fp8:
+            pool += [torch.full((nblk, bs, hkv, dh), 7, dtype=torch.uint8, device=device) for _ in range(2)]
+            pool += [torch.full((nblk, bs, hkv), 9.0, device=device) for _ in range(2)]
+        else:
+            pool += [torch.full((nblk, bs, hkv, dh), x, dtype=torch.bfloat16, device=device) for x in (3.0, -3.0)]
+    common = dict(num_kv_heads=hkv, num_prefill=1, prefill_cu_q=cu, prefill_cu_k=cu, max_q=length, max_k=length, k=k, v=v)
+    store_kvcache(k, v, a[0], a[1], slots, *a[2:])
+    outs = [torch.zeros(rows, hq, dh, dtype=torch.bfloat16, device=device) for _ in range(2)]
+    paged_attention(q, None, None, dh ** -0.5, out=outs[0], **common)
+    paged_attention(q, b[0], b[1], dh ** -0.5, out=outs[1], k_scale=b[2] if fp8 else None,
+                    v_scale=b[3] if fp8 else None, store_slot_mapping=slots, new_k=k, new_v=v, **common)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    for x, y in zip(a, b):
+        assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
