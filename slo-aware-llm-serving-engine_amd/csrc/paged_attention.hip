@@ -983,17 +983,18 @@ __device__ __forceinline__ void decode_final(const Params& p, int b, int h, int 
 // pieces then its V pieces): each copied to the row's slot (slots < 0 or past
 // the pool are skipped), all loads of the call first, then the stores; the
 // E4M3FN pool gets the quantising store of slo_store_kvcache.  Thread tid
-// takes pieces first + tid + j * NT (j < 4); with first a multiple of 16, the
-// 16 lanes of one (token, kv head) vector are whole groups.
-template <bool FP8>
+// takes pieces first + tid + j * NT (j < PIECES); with first a multiple of 16, the
+// 16 lanes of one (token, kv head) vector are whole groups.  LANDED: every load
+// this wavefront has issued so far has landed before the first store goes out.
+template <bool FP8, int PIECES = 4, bool LANDED = false>
 __device__ __forceinline__ void store_new_rows(const Params& p, int64_t first, int64_t end, int tid) {
   const int row = p.hkv * HD;  // elements of one K (or V) row
   const int per_tok = 2 * (row / 8);
-  for (int64_t i0 = first; i0 < end; i0 += 4 * NT) {
-    u32x4 x[4];
-    int64_t dst[4];
+  for (int64_t i0 = first; i0 < end; i0 += PIECES * NT) {
+    u32x4 x[PIECES];
+    int64_t dst[PIECES];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < PIECES; ++j) {
       const int64_t i = i0 + tid + j * NT;
       const int64_t t = i / per_tok;
       const int pc = (int)(i % per_tok);
@@ -1007,8 +1008,9 @@ __device__ __forceinline__ void store_new_rows(const Params& p, int64_t first, i
         if (slot >= 0 && slot < p.num_slots) dst[j] = 2 * (slot * row + e) + (isv ? 1 : 0);
       }
     }
+    if constexpr (LANDED) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < PIECES; ++j) {
       if constexpr (FP8) {
         // The 16 lanes of one (token, kv head) vector (whole groups: pieces
         // and the token are the same across them) share its amax.
@@ -1339,9 +1341,13 @@ __device__ void decode_run(const Params& p, Smem& sm, uint8_t* st0, uint8_t* st1
 // flight, then the cross-wavefront merge and, with several chunks in the
 // row, the split-K merge by the chunk whose ticket increment arrives last
 // (records of chunk c of (row, head) at dfirst + c * hkv).  mid() runs once
-// after the first steps' loads are issued; it returns whether it issued
-// memory operations of its own (the first wait then covers everything).
+// after the first two steps' loads are issued and says what it did to them:
+// SIDE_OPS, memory operations of its own followed them (the first wait then
+// covers everything), or SIDE_LANDED, it has waited for them itself (neither
+// step waits, so the stores that mid() issued last are not waited for before
+// the first key is used).
 // Ends with LDS free for the next chunk.
+enum Side : int { SIDE_NONE = 0, SIDE_OPS = 1, SIDE_LANDED = 2 };
 template <bool FP8, bool FOLD, typename Mid>
 __device__ __forceinline__ void run_chunk(const Params& p, Smem& sm, uint8_t* stage0, uint8_t* stage1, uint8_t* qbuf,
                                           const int* entries, const DMeta& m, int nrun, int nch, int dfirst, int tid,
@@ -1370,7 +1376,7 @@ __device__ __forceinline__ void run_chunk(const Params& p, Smem& sm, uint8_t* st
   uint8_t* nb = qbuf + QBUF + 2048 + wave * 512;
   decode_issue<FP8, FOLD>(p, sa, ca, na, step(0), 0, wave, lane);
   if (nrun > 1) decode_issue<FP8, FOLD>(p, sb, cb, nb, step(1), 0, wave, lane);
-  const bool side = mid();
+  const Side side = mid();
   const int n = lane & 15, g = lane >> 4;
   u32x4 qv[4];
   {
@@ -1385,7 +1391,8 @@ __device__ __forceinline__ void run_chunk(const Params& p, Smem& sm, uint8_t* st
   const int L = decode_L(p, m);
   for (int s = 0; s < nrun; ++s) {
     const bool odd = s & 1;
-    if (s + 1 < nrun && !(s == 0 && side)) __builtin_amdgcn_s_waitcnt(vmcnt_imm(GROUP));
+    if (s < 2 && side == SIDE_LANDED) asm volatile("" ::: "memory");
+    else if (s + 1 < nrun && !(s == 0 && side == SIDE_OPS)) __builtin_amdgcn_s_waitcnt(vmcnt_imm(GROUP));
     else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     const DMeta ms = step(s);
     decode_wstep<FP8, FOLD>(p, odd ? sb : sa, odd ? cb : ca, odd ? nb : na, decode_ntok<FP8>(p, ms, 0, wave),
@@ -1438,22 +1445,32 @@ __global__ void __launch_bounds__(NT, 2) decode_direct_kernel(Params p, int nch_
   const int x = blockIdx.x;
 
   // Once per workgroup, on every path (after the item's loads are issued
-  // where it has one): its share of the KV write (4 * NT pieces per
+  // where it has one): its share of the KV write (PIECES * NT pieces per
   // workgroup and turn: a launch may have many more query rows, each with a
   // new row, than decode rows) and of the zeros for query rows past every
-  // decode and prefill row.
+  // decode and prefill row.  The workgroups that write hold the first rows'
+  // first chunks, whose merges wait for them, so what they spend before the
+  // first key is on the launch's chain where such a row is the last to end:
+  // a quantising thread takes one piece (four took 2 us), and no step waits
+  // for the write's acknowledgement.  us for 8 layers, E4M3FN, as the store
+  // kernel and a launch / four pieces and the wait / now: 4 rows of 20-128
+  // tokens 60 / 66 / 50, 8 rows of 100-1,024 99 / 104 / 87, 16 rows of
+  // 512-4,096 257 / 242 / 242; where no such row ends last the four pieces
+  // were up to 5% faster (8 rows of 64-512 tokens 94 / 80 / 83).  bf16, four
+  // pieces with / without the wait: 4 rows of 64-512 tokens 79.2 / 76.6.
   auto side_work = [&]() {
-    bool any = false;
+    Side done = SIDE_NONE;
     if constexpr (FOLD) {
-      const int64_t per_wg = 4 * NT, all = (int64_t)p.nnew * (2 * (p.hkv * HD / 8));
+      constexpr int PIECES = FP8 ? 1 : 4;
+      const int64_t per_wg = PIECES * NT, all = (int64_t)p.nnew * (2 * (p.hkv * HD / 8));
       for (int64_t i = (int64_t)x * per_wg; i < all; i += (int64_t)gridDim.x * per_wg) {
-        store_new_rows<FP8>(p, i, min(all, i + per_wg), tid);
-        any = true;
+        store_new_rows<FP8, PIECES, true>(p, i, min(all, i + per_wg), tid);
+        done = SIDE_LANDED;
       }
     }
     const int64_t covered = (int64_t)p.q_off_prefill + (p.np_all > 0 ? max(p.cu_q_all[p.np_all], 0) : 0);
     if (covered < p.num_q_rows) {
-      any = true;
+      done = SIDE_OPS;
       const int per_row = p.hkv * p.G * HD / 8;
       const int64_t pieces = (p.num_q_rows - covered) * per_row;
       for (int64_t i = (int64_t)x * NT + tid; i < pieces; i += (int64_t)gridDim.x * NT) {
@@ -1461,7 +1478,7 @@ __global__ void __launch_bounds__(NT, 2) decode_direct_kernel(Params p, int nch_
         *reinterpret_cast<u32x4*>(p.out + row * p.out_stride + 8 * (i % per_row)) = u32x4{0, 0, 0, 0};
       }
     }
-    return any;
+    return done;
   };
 
   // With `spread` (bf16 pools, kv heads a multiple of the 8 XCDs, at most

@@ -485,3 +485,48 @@ def test_cold_launch_writes_rows_outside_every_prefill_row(device, fp8, head, le
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     for x, y in zip(a, b):
         assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens", [[1], [64, 65], [128, 129, 256, 257], [255, 1, 512, 513, 640, 2, 768, 769, 1025],
+                                  [37 * i % 300 + 1 for i in range(70)]])
+@pytest.mark.parametrize("views", ["v", "k", ""])
+def test_decode_folds_at_the_edges_of_a_step(device, fp8, lens, views):
+    # The workgroups that carry the write skip the waits of their first two
+    # steps: rows of one, two, three and more steps, one token short of a step,
+    # at it and past it.  As Qwen3 hands them over, K is contiguous and V a view
+    # of the QKV projection ("v"); the other way round ("k") the strides differ
+    # as well.  Output and pool bytes of the store kernel followed by the launch.
+    g = torch.Generator().manual_seed(len(lens))
+    rows, hq, hkv, dh, bs = len(lens), 32, 8, 128, 256
+    per = [(n + bs - 1) // bs for n in lens]
+    nblk = sum(per) + 1
+    perm = torch.randperm(nblk, generator=g).tolist()
+    tables, at = [], 0
+    for n in per:
+        tables.append(perm[at:at + n] + [-1] * (max(per) - n))
+        at += n
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)  # noqa: E731
+    slots = i32([t[(n - 1) // bs] * bs + (n - 1) % bs for t, n in zip(tables, lens)])
+    padded, dl = i32(tables), i32(lens)
+    qkv = torch.randn(rows, (hq + 2 * hkv) * dh, generator=g).to(torch.bfloat16).to(device)
+    q, k, v = (t.view(rows, -1, dh) for t in qkv.split([hq * dh, hkv * dh, hkv * dh], -1))
+    q, k, v = q.contiguous(), k if views == "k" else k.contiguous(), v if views == "v" else v.contiguous()
+    reserve_workspace(device, rows, max(per) * bs, hq, hkv, dh)
+    base = torch.randn(2, nblk * bs, hkv, dh, generator=g).to(torch.bfloat16).to(device)
+    ctx = SimpleNamespace(mixed=MixedAttentionContext(rows, 0, dl, padded, None, None, None, 0, 0), slot_mapping=slots)
+    outs, pools = [], []
+    for store in (_two_launch_store, store_kvcache):
+        if fp8:
+            pool = [torch.empty(nblk, bs, hkv, dh, dtype=torch.uint8, device=device) for _ in range(2)]
+            pool += [torch.empty(nblk, bs, hkv, device=device) for _ in range(2)]
+            every = torch.arange(nblk * bs, dtype=torch.int32, device=device)
+            store_kvcache(base[0], base[1], pool[0], pool[1], every, *pool[2:])
+        else:
+            pool = [base[i].clone().view(nblk, bs, hkv, dh) for i in range(2)]
+        outs.append(forward_mixed(q, k, v, pool[0], pool[1], ctx, dh ** -0.5, store, *pool[2:]))
+        pools.append(pool)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    for a, b in zip(*pools):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
