@@ -2726,6 +2726,11 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
         (reinterpret_cast<uintptr_t>(a->new_v) % 16))
       return fail(SLO_ERR_INVALID,
                   "paged_attention: new K/V must be contiguous 16-byte aligned bf16 rows, one per query row");
+    // (Scales of an E4M3FN pool, the pool's alignment: whichever kernel writes.)
+    const int rc = check_store(a->new_k, a->new_k_row_stride, a->new_v, a->new_v_row_stride, a->store_slot_mapping,
+                               a->num_new_rows, a->num_kv_heads, HD, a->kv_dtype, a->k_cache, a->v_cache, a->k_scale,
+                               a->v_scale, a->store_scale_floor);
+    if (rc) return rc;
   }
   if (store && !fold && !cold) {
     const int rc = slo_store_kvcache(a->new_k, a->new_k_row_stride, a->new_v, a->new_v_row_stride,

@@ -52,16 +52,10 @@ store_kvcache_kernel(const uint16_t* __restrict__ key, int64_t key_stride,
   }
 }
 
-}  // namespace slo
-
-using namespace slo;
-
-extern "C" int slo_store_kvcache(const void* key, int64_t key_row_stride, const void* value,
-                                 int64_t value_row_stride, const int32_t* slot_mapping,
-                                 int32_t num_tokens, int32_t num_kv_heads, int32_t head_dim,
-                                 int32_t kv_dtype, void* k_cache, void* v_cache, float* k_scale,
-                                 float* v_scale, int64_t num_slots, float scale_floor,
-                                 slo_stream_t stream) {
+int check_store(const void* key, int64_t key_row_stride, const void* value, int64_t value_row_stride,
+                const int32_t* slot_mapping, int32_t num_tokens, int32_t num_kv_heads, int32_t head_dim,
+                int32_t kv_dtype, const void* k_cache, const void* v_cache, const float* k_scale, const float* v_scale,
+                float scale_floor) {
   if (num_tokens < 0 || num_kv_heads <= 0) return fail(SLO_ERR_INVALID, "store_kvcache: bad token/head count");
   if (head_dim != 64 && head_dim != 128 && head_dim != 256)
     return fail(SLO_ERR_UNSUPPORTED, "store_kvcache: head_dim must be 64, 128 or 256");
@@ -75,6 +69,23 @@ extern "C" int slo_store_kvcache(const void* key, int64_t key_row_stride, const 
       (reinterpret_cast<uintptr_t>(v_cache) % 16))
     return fail(SLO_ERR_INVALID, "store_kvcache: rows must be 16-byte aligned (stride multiple of 8 elements)");
   if (2 * num_kv_heads * (head_dim / 8) > 65536) return fail(SLO_ERR_UNSUPPORTED, "store_kvcache: too many heads");
+  return SLO_OK;
+}
+
+}  // namespace slo
+
+using namespace slo;
+
+extern "C" int slo_store_kvcache(const void* key, int64_t key_row_stride, const void* value,
+                                 int64_t value_row_stride, const int32_t* slot_mapping,
+                                 int32_t num_tokens, int32_t num_kv_heads, int32_t head_dim,
+                                 int32_t kv_dtype, void* k_cache, void* v_cache, float* k_scale,
+                                 float* v_scale, int64_t num_slots, float scale_floor,
+                                 slo_stream_t stream) {
+  const int rc = check_store(key, key_row_stride, value, value_row_stride, slot_mapping, num_tokens, num_kv_heads,
+                             head_dim, kv_dtype, k_cache, v_cache, k_scale, v_scale, scale_floor);
+  if (rc) return rc;
+  if (num_tokens == 0) return SLO_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid(num_tokens), block(256);
   const auto* k16 = static_cast<const uint16_t*>(key);

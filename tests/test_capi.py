@@ -105,3 +105,40 @@ def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libslo_attn.so")
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         _lib.load()
+
+
+@pytest.mark.parametrize("shape", ["cold", "paged", "decode"])
+def test_kv_write_arguments_are_checked_on_every_path(shape):
+    # The launch may write the pool itself (cold prefill rows, decode rows) or
+    # through the store kernel (prefill rows with tables): each refuses an
+    # E4M3FN pool without scales and a pool off the 16-byte boundary before any
+    # pointer is touched (none of them is real).
+    lib = _lib.load()
+
+    def call(**over):
+        args = _lib.PagedAttentionArgs()
+        args.head_dim, args.num_heads, args.num_kv_heads, args.softmax_scale = 128, 32, 8, 0.1
+        args.q = args.out = args.k_cache = args.v_cache = args.new_k = args.new_v = args.store_slot_mapping = 4096
+        args.q_row_stride = args.out_row_stride = 32 * 128
+        args.num_q_rows = args.num_new_rows = 4
+        args.new_k_row_stride = args.new_v_row_stride = 8 * 128
+        args.num_blocks, args.block_size, args.phases = 2, 256, 3
+        args.kv_dtype, args.k_scale, args.v_scale, args.store_scale_floor = 1, 4096, 4096, 2.0 ** -64
+        args.workspace, args.workspace_bytes = 8192, 16  # too small: the first check after the KV write's
+        if shape == "decode":
+            args.num_decode, args.decode_lens, args.decode_tables = 4, 4096, 4096
+            args.decode_table_stride = args.decode_table_width = 1
+        else:
+            args.num_prefill, args.prefill_cu_q, args.prefill_cu_k, args.max_q, args.max_k = 1, 4096, 4096, 4, 4
+            args.k = args.v = 4096
+            args.k_row_stride = args.v_row_stride = args.num_kv_rows = 8 * 128
+            if shape == "paged":
+                args.prefill_tables, args.prefill_table_stride, args.prefill_table_width = 4096, 1, 1
+        for name, value in over.items():
+            setattr(args, name, value)
+        return lib.slo_paged_attention(ctypes.byref(args), None), lib.slo_last_error().decode()
+
+    for over, word in ((dict(k_scale=None), "scale"), (dict(v_scale=None), "scale"), (dict(k_cache=4104), "aligned"),
+                       (dict(v_cache=4104), "aligned"), (dict(kv_dtype=0, v_cache=4104), "aligned")):
+        code, message = call(**over)
+        assert code == 1 and word in message, (over, code, message)
