@@ -73,6 +73,9 @@ class MixedStepBuffers:
             raise ValueError("step does not fit this bucket")
         if len(tables) != d + r or any(len(t) > self.width for t in tables):
             raise ValueError("one block table per row, at most table_width entries")
+        if len(input_ids) < d:
+            # (A slice assignment would give one id to every decode row.)
+            raise IndexError(f"{len(input_ids)} input ids for {d} decode rows")
         rows = self.dc + self.pc
         ids, h = self._ids, self._words
         self._copied.synchronize()  # the previous step's copy has left the pinned buffer
