@@ -24,7 +24,7 @@ from torch import nn
 from . import _lib
 from .context import get_context
 from .mixed_attention import forward_mixed
-from .ops import check_store, foldable, foldable_strided, paged_attention, store_kvcache
+from .ops import check_store, foldable, folds_alone, paged_attention, store_kvcache
 
 __all__ = ["Attention", "store_kvcache"]
 
@@ -64,8 +64,8 @@ class Attention(nn.Module):
         # only; otherwise the store kernel runs first.
         paged = context.is_prefill and context.block_tables is not None
         fold = have_cache and not kv_stored and (
-            self.k_scale is None and foldable(k, v) if paged
-            else foldable_strided(k, v) and (self.k_scale is None or q.shape[1] <= 8 * k.shape[1]))
+            (self.k_scale is None and foldable(k, v))
+            or (not paged and folds_alone(q, k, v, k_cache, self.k_scale)))
         if fold:
             check_store(k, v, k_cache, v_cache, context.slot_mapping, *self._scales())
         elif have_cache and not kv_stored:

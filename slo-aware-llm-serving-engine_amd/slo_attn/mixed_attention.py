@@ -14,7 +14,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .ops import check_store, foldable, foldable_strided, paged_attention, store_kvcache
+from .ops import check_store, foldable, folds_alone, paged_attention, store_kvcache
 
 
 @dataclass
@@ -60,8 +60,9 @@ def forward_mixed(q, k, v, k_cache, v_cache, context, scale, store_fn,
     # pool), also fold rows that are views of the QKV projection.
     alone = not meta.num_prefill_tokens or (not meta.num_decode and not meta.prefill_has_history)
     fold = (store_fn is store_kvcache and phases == _lib.PHASE_ALL
-            and (foldable_strided(k, v) if alone else foldable(k, v))
-            and (k_scale is None or (q.shape[1] <= 8 * k.shape[1] and alone)))
+            and ((foldable(k, v)
+                  and (k_scale is None or (q.shape[1] <= 8 * k.shape[1] and not meta.num_prefill_tokens)))
+                 or (alone and folds_alone(q, k, v, k_cache, k_scale))))
     if fold and alone:
         phases |= _lib.NEW_ROWS_STRIDED
     if fold:

@@ -98,15 +98,27 @@ def foldable(key: torch.Tensor, value: torch.Tensor) -> bool:
 
 
 def foldable_strided(key: torch.Tensor, value: torch.Tensor) -> bool:
-    """Whether a launch without prefill rows can carry the KV write of these
-    new rows (``_lib.NEW_ROWS_STRIDED``): bf16 ``[N, num_kv_heads, head_dim]``
-    rows of contiguous heads on 16-byte boundaries, such as the K and V views
-    of a fused QKV projection's output."""
+    """Whether a launch without prefill rows, or of cold prefill rows only, can
+    carry the KV write of these new rows (``_lib.NEW_ROWS_STRIDED``): bf16
+    ``[N, num_kv_heads, head_dim]`` rows of contiguous heads on 16-byte
+    boundaries, such as the K and V views of a fused QKV projection's output."""
     if key.dim() != 3 or key.dtype != torch.bfloat16 or value.dtype != torch.bfloat16:
         return False
     row, d = key.shape[1] * key.shape[2], key.shape[2]
     return all(t.stride(2) == 1 and t.stride(1) == d and t.stride(0) >= row and t.stride(0) % 8 == 0
                and t.data_ptr() % 16 == 0 for t in (key, value))
+
+
+def folds_alone(q: torch.Tensor, key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
+                k_scale: torch.Tensor | None) -> bool:
+    """Whether a launch of decode rows only, or of cold prefill rows only,
+    carries the KV write of ``key``/``value``: ``foldable_strided`` rows, one
+    per query row, into a 4-dimensional pool view; with an E4M3FN pool at most
+    8 query heads per kv head.  Everything else (keys of a whole cold row
+    beside the queries of its last tokens, a pool view of merged heads) keeps
+    the store kernel's own launch, which takes it."""
+    return (key.dim() == 3 and key.shape[0] == q.shape[0] and k_cache.dim() == 4 and foldable_strided(key, value)
+            and (k_scale is None or q.shape[1] <= 8 * key.shape[1]))
 
 
 def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,

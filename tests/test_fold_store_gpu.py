@@ -530,3 +530,56 @@ def test_decode_folds_at_the_edges_of_a_step(device, fp8, lens, views):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     for a, b in zip(*pools):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("case", ["tail queries", "more new rows than decode rows", "merged heads"])
+def test_v0_steps_that_no_launch_carries(device, fp8, case):
+    # V0 steps with views of the QKV projection that keep the store kernel's own
+    # launch: the queries of a cold prompt's last tokens beside the keys of all
+    # of it, decode steps with more new rows than query rows, and a cold step on
+    # a pool view of merged heads.  Output and pool bytes of the store kernel
+    # followed by the attention launch.
+    g = torch.Generator().manual_seed(17)
+    hq, hkv, dh, bs, nblk, n = 32, 8, 128, 256, 3, 100
+    qkv = torch.randn(n, (hq + 2 * hkv) * dh, generator=g).to(torch.bfloat16).to(device)
+    q, k, v = (t.view(n, -1, dh) for t in qkv.split([hq * dh, hkv * dh, hkv * dh], -1))
+    q = q.contiguous()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)  # noqa: E731
+    slots = torch.randperm(nblk * bs, generator=g)[:n].to(torch.int32).to(device)
+    decode = case.startswith("more")
+    rows = 100 if case.startswith("merged") else 20
+    q = q[-rows:]
+    lens, tables = i32([5 + i for i in range(rows)]), i32([[i % nblk] for i in range(rows)])
+    cu_q, cu_k = i32([0, rows]), i32([0, n])
+    outs, pools = [], []
+    for fold in (False, True):
+        if fp8:
+            pool = [torch.full((nblk, bs, hkv, dh), 7, dtype=torch.uint8, device=device) for _ in range(2)]
+            pool += [torch.full((nblk, bs, hkv), 0.5, device=device) for _ in range(2)]
+        else:
+            pool = [torch.full((nblk, bs, hkv, dh), x, dtype=torch.bfloat16, device=device) for x in (3.0, -3.0)]
+        if not fold:
+            store_kvcache(k, v, pool[0], pool[1], slots, *pool[2:])
+            where = (dict(num_decode=rows, decode_lens=lens, decode_tables=tables, k_scale=pool[2] if fp8 else None,
+                          v_scale=pool[3] if fp8 else None) if decode else
+                     dict(num_prefill=1, prefill_cu_q=cu_q, prefill_cu_k=cu_k, max_q=rows, max_k=n, k=k, v=v))
+            outs.append(paged_attention(q, pool[0] if decode else None, pool[1] if decode else None, dh ** -0.5,
+                                        num_kv_heads=hkv, **where))
+        else:
+            attn = Attention(hq, dh, dh ** -0.5, hkv)
+            merged = case.startswith("merged")
+            attn.k_cache, attn.v_cache = (p.view(nblk, bs, -1) if merged else p for p in pool[:2])
+            if fp8:
+                attn.k_scale, attn.v_scale = pool[2:]
+            if decode:
+                set_context(False, slot_mapping=slots, context_lens=lens, block_tables=tables)
+            else:
+                set_context(True, cu_q, cu_k, rows, n, slots)
+            outs.append(attn(q, k, v).view(rows, hq, dh))
+            reset_context()
+        pools.append(pool)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    for a, b in zip(*pools):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
