@@ -301,12 +301,19 @@ void launch_lm(dim3 grid, hipStream_t s, const uint16_t* hidden, int64_t hstride
   // chunks fit the LDS; row offsets within a block are 32 bits): 151,936 x
   // 2,560 at 1, 26 and 64 rows 139 -> 122, 148 -> 131, 165 -> 145 us; 33,333 x
   // 1,024 at 26 rows 26.6 -> 24.1 us.  Weight rows a multiple of 8 KiB apart
-  // put a chunk of every row on the same memory channels: up to 32 sampled
-  // rows the register kernel's 512-byte chunks are faster there (151,936 x
-  // 4,096 at 26 rows 242 against 251 us, 32,000 x 4,096 at one row 61 against
-  // 63), above them the stream again (100,003 x 4,096 at 60 rows 195 -> 186).
+  // put a chunk of every row on the same memory channels, where the register
+  // kernel's 512-byte chunks are faster up to 32 sampled rows (151,936 x 4,096
+  // at 26 rows 242 against 251 us, 32,000 x 4,096 at one row 61 against 63).
+  // Above that it stays faster with rows of exactly 16 KiB, and up to 48 sampled
+  // rows of 8 KiB (us, register / stream: 33-48 rows, 32,000 x 4,096 55 / 62,
+  // 151,936 x 4,096 255 / 262, 60,000 x 8,192 200 / 237; 49-64 rows, 60,000 x
+  // 8,192 228 / 235), and loses beyond (33-48 rows, 60,000 x 12,288 307 / 270,
+  // 40,000 x 16,384 328 / 264, 40,000 x 20,480 450 / 351; 49-64 rows, 151,936 x
+  // 4,096 279 / 271, 60,000 x 12,288 325 / 281).
   if constexpr (NCT <= 4) {
-    if (wstride < (1 << 23) && hstride < (1 << 23) && (wstride % 4096 != 0 || NCT > 2)) {
+    const bool same_channels =
+        wstride % 4096 == 0 && (NCT <= 2 || wstride == 8192 || (NCT == 3 && wstride == 4096));
+    if (wstride < (1 << 23) && hstride < (1 << 23) && !same_channels) {
       const dim3 sgrid(std::min<unsigned>(grid.x, (unsigned)cus));
       hipLaunchKernelGGL((lm_head_stream_kernel<NCT>), sgrid, dim3(256), 0, s, hidden, hstride, M, w, wstride, V, H,
                          logits, lstride, keys);

@@ -40,7 +40,7 @@ def _check_tokens(tokens, ref_logits_bits):
 
 # Up to 64 rows the weight streams through LDS in 128-row blocks of 128-column
 # chunks (one chunk per row, a ragged last block, more blocks than workgroups);
-# 8 KiB weight rows keep the register kernel up to 32 rows.
+# 8 KiB weight rows keep the register kernel up to 48 rows.
 @pytest.mark.parametrize("rows,vocab,hidden", [(1, 1000, 128), (7, 5003, 512), (65, 3000, 2560), (128, 777, 256),
                                                (16, 129, 256), (17, 70001, 128), (33, 34000, 384), (64, 127, 640),
                                                (32, 300, 4096), (40, 300, 4096)])
@@ -86,3 +86,21 @@ def test_rejects_bad_arguments(device):
         lm_head_argmax(h[:, :200].contiguous(), w[:, :200].contiguous())
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         lm_head_argmax(h.cpu(), w.cpu())
+
+
+# Weight rows a multiple of 8 KiB apart choose between the two kernels by the
+# sampled rows and the distance: both sides of each edge, and rows that are a
+# part of a longer one.
+@pytest.mark.parametrize("rows,hidden,stride", [(32, 4096, 4096), (33, 4096, 4096), (48, 256, 8192), (49, 256, 8192),
+                                                (33, 256, 12288), (32, 256, 12288), (40, 384, 4096)])
+def test_weight_rows_on_the_same_channels(device, rows, hidden, stride):
+    g = torch.Generator().manual_seed(rows + stride)
+    vocab = 300
+    h = torch.randn(rows, hidden, generator=g).to(torch.bfloat16)
+    w = torch.randn(vocab, stride, generator=g).to(torch.bfloat16).to(device)[:, :hidden]
+    tokens, logits = lm_head_argmax(h.to(device), w, return_logits=True)
+    want = _f(lm_head.logits(_bits(h), _bits(w)))
+    got = _f(_bits(logits))
+    ulp = np.ldexp(1.0, np.frexp(np.abs(want) + 1e-30)[1] - 8)
+    assert (np.abs(got - want) <= ulp + 1e-6 * np.abs(want).max()).all()
+    assert np.array_equal(tokens.cpu().numpy(), np.argmax(got, axis=1))
