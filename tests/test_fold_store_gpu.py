@@ -16,7 +16,8 @@ import torch
 from slo_attn import (Attention, MixedAttentionContext, forward_mixed, reserve_workspace, reset_context,
                       set_context, store_kvcache)
 import workloads
-from slo_attn.ops import paged_attention
+from slo_attn import _lib
+from slo_attn.ops import paged_attention, workspace_events
 from types import SimpleNamespace
 
 pytestmark = pytest.mark.gpu
@@ -583,3 +584,97 @@ def test_v0_steps_that_no_launch_carries(device, fp8, case):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     for a, b in zip(*pools):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def _cold_launch_against_store(device, fp8, cu_q, cu_k, hq, hkv, seed, views="v"):
+    """A cold prefill launch with the KV write (keys from the contiguous rows
+    k/v, which may be longer than the new rows) against the store kernel and
+    the same launch without it."""
+    g = torch.Generator().manual_seed(seed)
+    dh, bs, n, keys = 128, 256, cu_q[-1], cu_k[-1]
+    nblk = (n + bs - 1) // bs + 2
+    slots = torch.randperm(nblk * bs, generator=g)[:n].to(torch.int32).to(device)
+    qkv = torch.randn(n, (hq + 2 * hkv) * dh, generator=g).to(torch.bfloat16).to(device)
+    q, nk, nv = (t.view(n, -1, dh) for t in qkv.split([hq * dh, hkv * dh, hkv * dh], -1))
+    q, nk, nv = q.contiguous(), nk if views == "k" else nk.contiguous(), nv if views == "v" else nv.contiguous()
+    k, v = nk, nv
+    if keys != n:
+        k, v = (torch.randn(keys, hkv, dh, generator=g).to(torch.bfloat16).to(device) for _ in range(2))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)  # noqa: E731
+    lq = [b - a for a, b in zip(cu_q, cu_q[1:])]
+    lk = [b - a for a, b in zip(cu_k, cu_k[1:])]
+    common = dict(num_kv_heads=hkv, num_prefill=len(lq), prefill_cu_q=i32(cu_q), prefill_cu_k=i32(cu_k), max_q=max(lq),
+                  max_k=max(lk), k=k, v=v)
+    reserve_workspace(device, 0, 0, hq, hkv, dh)
+    outs, pools = [], []
+    for fold in (False, True):
+        if fp8:
+            pool = [torch.full((nblk, bs, hkv, dh), 7, dtype=torch.uint8, device=device) for _ in range(2)]
+            pool += [torch.full((nblk, bs, hkv), 9.0, device=device) for _ in range(2)]
+        else:
+            pool = [torch.full((nblk, bs, hkv, dh), x, dtype=torch.bfloat16, device=device) for x in (3.0, -3.0)]
+        if fold:
+            outs.append(paged_attention(q, pool[0], pool[1], dh ** -0.5, k_scale=pool[2] if fp8 else None,
+                                        v_scale=pool[3] if fp8 else None, store_slot_mapping=slots, new_k=nk, new_v=nv,
+                                        phases=_lib.PHASE_ALL | _lib.NEW_ROWS_STRIDED, **common))
+        else:
+            store_kvcache(nk, nv, pool[0], pool[1], slots, *pool[2:])
+            outs.append(paged_attention(q, None, None, dh ** -0.5, **common))
+        pools.append(pool)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    for a, b in zip(*pools):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    return q, k, v, outs[1], lq, lk
+
+
+def _cu(lens):
+    out = [0]
+    for n in lens:
+        out.append(out[-1] + n)
+    return out
+
+
+def _plain_prefill(q, k, v, lq, lk):
+    out, a, b = [], 0, 0
+    for m, n in zip(lq, lk):
+        s = torch.einsum("qhd,khd->hqk", q[a:a + m].float().cpu(),
+                         k[b:b + n].float().cpu().repeat_interleave(q.shape[1] // k.shape[1], 1)) * q.shape[2] ** -0.5
+        s.masked_fill_(torch.arange(n) > torch.arange(m)[:, None] + n - m, float("-inf"))
+        out.append(torch.einsum("hqk,khd->qhd", s.softmax(-1),
+                                v[b:b + n].float().cpu().repeat_interleave(q.shape[1] // v.shape[1], 1)))
+        a, b = a + m, b + n
+    return torch.cat(out)
+
+
+# The item orders of a cold launch: ranked units up to 128 rows, 1,024 units and
+# 16,384 units x rows, row order past each of these, and a row split in two key
+# ranges (more keys than queries, 32-position blocks whose second part stores
+# nothing).  Empty rows and ties between equal rows among them.
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("name,lens,hist,hkv", [
+    ("128 rows", [(5 * i) % 33 for i in range(128)], 0, 4),
+    ("129 rows", [(5 * i) % 33 for i in range(129)], 0, 4),
+    ("140 equal and empty rows", [0, 33] * 70, 0, 4),
+    ("128 rows, more than 16,384 units x rows", [(7 * i) % 41 for i in range(128)], 0, 4),
+    ("1,021 units of 16 positions", [4096] + [816] * 15, 0, 1),
+    ("1,036 units of 16 positions", [4096] + [832] * 15, 0, 1),
+    ("split row", [96, 40], 1500, 4),
+    ("split row of 33 queries", [33, 1, 64], 2100, 4),
+])
+def test_cold_write_in_every_item_order(device, fp8, name, lens, hist, hkv):
+    # Qwen3's pair: K contiguous, V a view of the projection.
+    cu_q = _cu(lens)
+    cu_k = _cu([n + (hist if i == 0 else 0) for i, n in enumerate(lens)])
+    q, k, v, out, lq, lk = _cold_launch_against_store(device, fp8, cu_q, cu_k, 4 * hkv, hkv, 5)
+    if hist:
+        assert workspace_events(device)["split_prefill_merges"] > 0
+    want = _plain_prefill(q, k, v, lq, lk)
+    assert (out.float().cpu() - want).abs().max() <= 2e-2
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("views", ["v", "k", ""])
+@pytest.mark.parametrize("lens,hq,hkv", [([1], 32, 8), ([31, 33, 1, 64, 100], 8, 8), ([700, 257], 64, 8)])
+def test_cold_write_with_different_k_and_v_strides(device, fp8, views, lens, hq, hkv):
+    _cold_launch_against_store(device, fp8, _cu(lens), _cu(lens), hq, hkv, 9, views)
