@@ -2077,6 +2077,7 @@ constexpr int MODES = 4;
 template <bool FP8, int MODE, bool FOLD = false>
 __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
   constexpr bool PF_ONLY = MODE == MODE_PREFILL || MODE == MODE_COLD;
+  static_assert(!(PF_ONLY && FOLD), "prefill-only launches write in MODE_COLD or after the store kernel");
   constexpr bool HAS_DEC = !PF_ONLY;
   // (The bf16 MODE_PREFILL instantiation spilled registers with the source
   // known; the E4M3FN one went from 256 to 239.)
@@ -2156,7 +2157,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
       w += __shfl_xor(w, d, 64);
       tm = max(tm, __shfl_xor(tm, d, 64));
       dn += __shfl_xor(dn, d, 64);
-      if constexpr (PF_ONLY && !FOLD) tu = max(tu, __shfl_xor(tu, d, 64));
+      if constexpr (PF_ONLY) tu = max(tu, __shfl_xor(tu, d, 64));
     }
     if (lane == 0) {
       sm.wsum[wave] = w;
@@ -2181,10 +2182,8 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
       // operand reads per query (three 512-token chunks after prefixes
       // 0/2048/512: 65.7 -> 51.3 us; two after 0 and 1,024: 38.0 -> 37.8
       // us); the other rows take 16 only when a row this long cannot split
-      // (tunsplit).  (A folded prefill-only instantiation would keep 16 for
-      // all: its 32-position split items spilled registers; launch_attention
-      // runs prefill-only launches without the KV write.)
-      if (FOLD || (int64_t)tunsplit * gridDim.x > 2 * wt) bq = 16;
+      // (tunsplit).
+      if ((int64_t)tunsplit * gridDim.x > 2 * wt) bq = 16;
     }
     // (E4M3FN launches always take full 512-token items: measured 27.0 ->
     // 25.5 us on 16 rows of 64-1024 tokens and 54 -> 51 us on 24 rows of
@@ -2239,9 +2238,9 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (i >= per || r0 + i >= nrows) continue;
-      // Split rows take 32-position blocks except in the folded instantiation.
+      // Split rows take 32-position blocks.
       const bool sp = pf_splits(p, r0 + i, tmr[i], sm.pf_split_thr);
-      const int c = cnt_a[i] + (bq == 16 && !(sp && !FOLD) ? cnt_d[i] : 0);
+      const int c = cnt_a[i] + (bq == 16 && !sp ? cnt_d[i] : 0);
       base_c += c;
       if (sp) extra_c += c;
     }
@@ -2258,8 +2257,8 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
     if (tid == 0) {
       const int all = sm.wsum[0] + sm.wsum[1] + sm.wsum[2] + sm.wsum[3];
       const int ext = sm.dsum[0] + sm.dsum[1] + sm.dsum[2] + sm.dsum[3];
-      // Record slots of 32-position items (16 in the folded instantiation).
-      const int cap = (int)(p.pf_split_bytes / (int64_t)(sizeof(float) * (size_t)PF_REC_FLOATS * (FOLD ? bq / 16 : 2)));
+      // Record slots of 32-position items.
+      const int cap = (int)(p.pf_split_bytes / (int64_t)(sizeof(float) * (size_t)PF_REC_FLOATS * 2));
       if (ext == 0 || all + ext > cap || all + ext > MAX_COUNTERS) sm.pf_split_thr = 1 << 30;
     }
     __syncthreads();
@@ -2273,7 +2272,7 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const bool sp = PF_ONLY && r0 + i < p.np && pf_splits(p, r0 + i, tmr[i], sm.pf_split_thr);
-    const bool alt = r0 + i < p.np ? ((bq == 16 && !(sp && !FOLD)) || tmr[i] > sm.split_tiles)
+    const bool alt = r0 + i < p.np ? ((bq == 16 && !sp) || tmr[i] > sm.split_tiles)
                                    : dchunk == d_chunk_min<FP8>();
     cnt[i] = cnt_a[i] + (alt ? cnt_d[i] : 0);
     if (sp) cnt[i] *= 2;
@@ -2439,17 +2438,14 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
             pf_work(p, r, wr, tr);
             sp = pf_splits(p, r, tr, sm.pf_split_thr);
           }
-          // Split items only where the row splits (32-position blocks, 16 in
-          // the folded instantiation); other items keep the tile loop
-          // compiled without the split's range and merge code.
+          // Split items only where the row splits (32-position blocks); other
+          // items keep the tile loop compiled without the split's range and
+          // merge code.
           const int lr = sorted ? (int)(pf_units[item / per_unit] & 0xffffu) * per_unit + item % per_unit
                                 : item - sm.off[r];
-          if (sp) {
-            if constexpr (!FOLD) prefill_item<FP8, 2, FOLD, true, SRC>(p, sm, stage0, stage1, r, lr, ltid, item, true);
-            else prefill_item<FP8, 1, FOLD, true, SRC>(p, sm, stage0, stage1, r, lr, ltid, item, true);
-          }
-          else if (bq == 16) prefill_item<FP8, 1, FOLD, false, SRC>(p, sm, stage0, stage1, r, lr, ltid);
-          else prefill_item<FP8, 2, FOLD, false, SRC>(p, sm, stage0, stage1, r, lr, ltid);
+          if (sp) prefill_item<FP8, 2, false, true, SRC>(p, sm, stage0, stage1, r, lr, ltid, item, true);
+          else if (bq == 16) prefill_item<FP8, 1, false, false, SRC>(p, sm, stage0, stage1, r, lr, ltid);
+          else prefill_item<FP8, 2, false, false, SRC>(p, sm, stage0, stage1, r, lr, ltid);
         } else if constexpr (HAS_PF) {
           // The row's items are 16-position blocks exactly when the item
           // counts above took them so (tmr > split_tiles, E4M3FN launches).
