@@ -488,7 +488,7 @@ def main():
         "roofline_qk_norm_rope_store": hbm(qk_bytes, t_qk, traffic=traffic_of("qk"), kernel="qk_norm_rope_store_kernel",
                                            algorithmic_bytes_per_launch=qk_bytes, avg_launch_us=round(t_qk, 2),
                                            tokens=tokens),
-        "roofline_lm_head_argmax": hbm(lm_bytes, t_lm, traffic=traffic_of("lm_head"), kernel="lm_head_argmax_kernel",
+        "roofline_lm_head_argmax": hbm(lm_bytes, t_lm, traffic=traffic_of("lm_head"), kernel="lm_head_stream_kernel",
                                        algorithmic_bytes_per_launch=lm_bytes, avg_launch_us=round(t_lm, 2),
                                        rows=sample_rows, vocab=vocab, hidden=hidden,
                                        torch_linear_argmax_us=round(t_lm_torch, 2)),

@@ -10,7 +10,8 @@
  * sized from shapes and capacities only, so calls may be recorded into a HIP
  * graph.
  *
- * Pool geometry (per layer), identical to the reference engine:
+ * Pool geometry (per layer), identical to the reference engine (K/V on 16-byte
+ * boundaries wherever a call writes them):
  *   K/V   [num_blocks, block_size, num_kv_heads, head_dim]  bf16, or E4M3FN
  *         bytes when kv_dtype == SLO_KV_FP8_E4M3FN
  *   scale [num_blocks, block_size, num_kv_heads]            fp32 (FP8 only)
@@ -212,11 +213,14 @@ typedef struct slo_paged_attention_args {
    * Lk - Lq of a prefill row read through prefill_tables is new row
    * num_decode + cu_q[r] + j - (Lk - Lq).  The result equals the separate
    * store followed by this launch, bit for bit; no slot written by the launch
-   * may be read through a table by it except as such a new token.  Launches
-   * without decode rows whose prefill rows have tables, and E4M3FN launches
-   * with decode and prefill rows, make that order themselves: the store
-   * kernel, then the attention launch (two kernels on `stream`, the same
-   * bytes and outputs). */
+   * may be read through a table by it except as such a new token (a decode
+   * row whose slot is not its last token's, or a second row of the same
+   * sequence, needs slo_store_kvcache first).  Launches without decode rows
+   * whose prefill rows have tables, and E4M3FN launches with decode and
+   * prefill rows, make that order themselves: the store kernel, then the
+   * attention launch (two kernels on `stream`, the same bytes and outputs).
+   * Launches of prefill rows without tables read no pool: their slots are
+   * free of that rule. */
   const int32_t* store_slot_mapping;  /* [num_new_rows] or NULL */
   const void* new_k;
   int64_t new_k_row_stride;

@@ -2,10 +2,12 @@
 //
 // Replaces the per-phase flash-attn calls of forward_mixed
 // (nanovllm/layers/mixed_attention.py:36-57) and of the V0 branches of
-// Attention.forward (nanovllm/layers/attention.py:68-78), and, with a bf16
-// pool, the KV write that precedes them (attention.py:10-40): the launch then
-// reads the step's new tokens from their rows and writes them to the pool as
-// tail work (FOLD instantiations).
+// Attention.forward (nanovllm/layers/attention.py:68-78), and the KV write that
+// precedes them (attention.py:10-40).  Three ways, chosen in launch_attention:
+// launches with decode rows read the step's new tokens from their rows and
+// write them to the pool as tail work (FOLD instantiations; E4M3FN pools only
+// without prefill rows); launches of cold prefill rows write them in their
+// items (MODE_COLD); every other launch follows the store kernel.
 //
 // Work list.  Every workgroup (4 wavefronts, two workgroups per CU) first
 // derives, from the metadata alone, the number of work items of every row and
@@ -2070,10 +2072,11 @@ enum Mode : int {
 
 constexpr int MODES = 4;
 
-// FOLD: the launch carries the KV write of the step's new tokens (bf16
-// pools): prefill tiles read new tokens from the new rows, and the tail tasks
-// include the store.  A separate instantiation, so launches without it keep
-// the prefill tile loop's smaller register footprint.
+// FOLD: a launch with decode rows carries the KV write of the step's new
+// tokens (bf16 pools; E4M3FN in MODE_DECODE): prefill tiles read new tokens
+// from the new rows, and the tail tasks include the store.  A separate
+// instantiation, so launches without it keep the prefill tile loop's smaller
+// register footprint.
 template <bool FP8, int MODE, bool FOLD = false>
 __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
   constexpr bool PF_ONLY = MODE == MODE_PREFILL || MODE == MODE_COLD;
@@ -2298,9 +2301,8 @@ __global__ void __launch_bounds__(NT, 2) paged_attention_kernel(Params p) {
   const int total = sm.off[nrows];
   const int decode_base = sm.off[p.np];
   // Prefill-only launches: rank the units by their block's key count (ties:
-  // lower row, then lower u, so the two halves of a split block stay adjacent
-  // and item + hkv * HG is the second half of item).  Items are numbered in
-  // that order instead of row by row, so every row's heaviest items start
+  // lower row, then lower u).  Items are numbered in that order instead of row
+  // by row, so every row's heaviest items start
   // first (four cold rows of 267-1,843 tokens: a later row's heaviest items
   // otherwise waited for the lighter items of the rows before it).
   const int per_unit = p.hkv * p.HG;
@@ -2542,8 +2544,8 @@ AttnKernel attn_kernel(bool fold, bool fp8, int mode) {
         paged_attention_kernel<true, MODE_DECODE>, nullptr}},
       // Prefill-only launches of rows with tables and E4M3FN launches with
       // decode and prefill rows never carry the KV write (launch_attention
-      // runs the store kernel first); launches of cold rows carry it in their
-      // own instantiation, FOLD or not.
+      // runs the store kernel first); launches of cold rows carry it in
+      // MODE_COLD above.
       {{paged_attention_kernel<false, MODE_MIXED, true>, nullptr, paged_attention_kernel<false, MODE_DECODE, true>,
         nullptr},
        {nullptr, nullptr, paged_attention_kernel<true, MODE_DECODE, true>, nullptr}},
@@ -2563,9 +2565,14 @@ DirectKernel direct_kernel(bool fold, bool fp8) {
 // run the work lists.  Measured on rows of 64-8192 tokens: the direct kernel
 // wins up to these sizes (16 rows of 64-1024 tokens 30 -> 15 us, 24 rows of
 // 256-4096 53 -> 51 us bf16 and 41 -> 37 us E4M3FN), the work lists beyond.
-// (E4M3FN, table width 4,096 tokens: 40 rows of 256-4,096, a grid of 2.5 times,
-// 56.0 -> 51.0 us; 48 rows of 512-4,096, 3 times, 61.4 -> 57.9; 64 rows, 4
-// times, 71.2 with the work lists against 76.0.)
+// (E4M3FN, each with the store kernel's launch before it, table width 4,096
+// tokens: 40 rows of 256-4,096, a grid of 2.5 times, 56.0 -> 51.0 us; 48 rows
+// of 512-4,096, 3 times, 61.4 -> 57.9; 64 rows, 4 times, 71.2 with the work
+// lists against 76.0.  Between two and three times at other widths and head
+// counts, us for 4 layers, work lists after the store kernel / direct with the
+// write: 190 rows at 1,024 tokens 257 / 218, 96 at 2,048 255 / 236, 24 at 8,192
+// 284 / 245, 12 at 16,384 290 / 207; 96 rows at 4,096 and 4 kv heads 252 / 234,
+// 24 at 16 kv heads 281 / 268; 40 rows of 64-1,024 in tables of 4,096 128 / 80.)
 constexpr int DIRECT_MAX_ROUNDS[2] = {4, 3};
 constexpr int DIRECT_CHUNK_MAX = 1024;  // tokens
 
@@ -2690,15 +2697,16 @@ int launch_attention(const slo_paged_attention_args* a, void* ws, size_t ws_byte
   }
   const bool store = a->store_slot_mapping != nullptr;
   // The KV write runs inside launches with decode rows except on E4M3FN
-  // pools with prefill rows; elsewhere it runs as the store kernel first and
-  // the launch reads the pool (same bytes and outputs).  The folded E4M3FN
+  // pools with prefill rows (`fold`), and inside launches of cold prefill rows
+  // only (`cold`); elsewhere it runs as the store kernel first and the launch
+  // reads the pool (same bytes and outputs).  The folded E4M3FN
   // instantiations with prefill rows spilled registers and measured slower
   // (108 against 72 us on 24 decode rows of 256-4096 tokens beside two
   // 512-token chunks); prefill-only launches without the write split their
-  // long rows' keys over 32-position blocks, which the folded instantiation
-  // cannot (three 512-token chunks after prefixes 0/2048/512: 74.7 -> 55.1 us
-  // for the step; four cold rows of 267-1,843 tokens 91.1 -> 90.1 us), while
-  // the mixed launch gains from the fold (65.5 against 70.6 us).
+  // long rows' keys over 32-position blocks, which a folded instantiation
+  // could not (three 512-token chunks after prefixes 0/2048/512: 74.7 -> 55.1
+  // us for the step), while the mixed launch gains from the fold (65.5 against
+  // 70.6 us).
   const bool fold = store && do_dec && !(fp8 && do_pf);
   // Prefill rows without tables read the contiguous K/V only: the launch's
   // items write the new rows to the pool (store_head_rows).

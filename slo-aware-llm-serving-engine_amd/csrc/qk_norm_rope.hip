@@ -27,9 +27,10 @@
 // square root and division are one refined v_rsq_f64, the sine is negated
 // once per token instead of choosing between two results per element, and
 // rows are addressed by a uniform base and a 32-bit offset: 9.6 -> 8.5 us for
-// 1,048 tokens, graph-replayed.  (384 threads, two heads in every group:
-// 9.1 us; 256 threads and three heads, before these changes, 10.0 against
-// 9.4 us; one head per group, 768 threads, 9.6 us.)
+// 1,048 tokens, the same buffers replayed; 10.8 -> 10.1 us where each of 8
+// layers has its own, read from HBM.  (On the same buffers, 384 threads, two
+// heads in every group, 9.1 us; before these changes 256 threads and three
+// heads 10.0 against 9.4 us, one head per group, 768 threads, 9.6 us.)
 #include "common.h"
 #include "capi_internal.h"
 
@@ -62,10 +63,13 @@ __device__ __forceinline__ double row_sum(double x) {
   x = add_dpp<0x141>(x);   // row_half_mirror
   return add_dpp<0x140>(x);  // row_mirror
 }
-// 1 / sqrt(x) rounded to fp32 from an fp64 value within about an ulp:
-// v_rsq_f64's 2^-23 refined once (third order) instead of the library's fp64
-// square root and division (about 50 instructions).  0, inf and NaN keep
-// v_rsq_f64's own result.
+// 1 / sqrt(x) rounded to fp32 from an fp64 value within about an ulp: with y
+// from v_rsq_f64 (2^-23) and e = 1 - x y^2, 1 / sqrt(x) = y (1 - e)^(-1/2), by
+// the series' terms up to e^2 (the next is below 2^-68), instead of the
+// library's fp64 square root and division (about 50 instructions).  Either way
+// is rounded twice, so the two agree unless the exact value lies within an
+// fp64 ulp of the middle of two fp32 values.  0, inf and NaN keep v_rsq_f64's
+// own result.
 __device__ __forceinline__ float rsqrt_rounded(float v) {
   const double x = (double)v;
   const double y = __builtin_amdgcn_rsq(x);

@@ -19,7 +19,7 @@ KV_FP8_E4M3FN = 1
 PHASE_DECODE = 1
 PHASE_PREFILL = 2
 PHASE_ALL = 3
-NEW_ROWS_STRIDED = 256  # or-ed into phases: strided new K/V rows (no prefill rows)
+NEW_ROWS_STRIDED = 256  # or-ed into phases: strided new K/V rows (decode rows only, or cold prefill rows only)
 FP8_SCALE_FLOOR = 2.0 ** -64
 NOALLOC_SCRATCH_BYTES = 64 << 20
 FP8_MAX = 448.0

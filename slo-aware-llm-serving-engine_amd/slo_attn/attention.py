@@ -56,12 +56,13 @@ class Attention(nn.Module):
         have_cache = bool(k_cache.numel() and v_cache.numel())
         # The pool is written inside the attention launch (same result, one
         # launch less) in decode steps, also from views of the QKV projection
-        # and into E4M3FN pools (at most 8 query heads per kv head): 16 rows of
-        # 64-1,024 tokens 18.1 -> 16.8 us a layer, 64 rows of 512-4,096 125.6
-        # -> 124.2 us, 40 E4M3FN rows of 256-4,096 51.3 -> 49.2 us.  So do cold
-        # prefill steps (no block tables), whose items write their own tokens.
-        # A prefill step that reads the pool hands over contiguous bf16 rows
-        # only; otherwise the store kernel runs first.
+        # and into E4M3FN pools (at most 8 query heads per kv head).  us a layer
+        # against the store kernel and a launch: 16 rows of 64-1,024 tokens 18.1
+        # -> 16.8, 64 rows of 512-4,096 125.6 -> 124.2; E4M3FN, both with the
+        # direct kernel, 40 rows of 256-4,096 51.3 -> 49.2, 4 rows of 20-128
+        # 7.5 -> 6.3.  So do cold prefill steps (no block tables), whose items
+        # write their own tokens.  A prefill step that reads the pool hands over
+        # contiguous bf16 rows only; otherwise the store kernel runs first.
         paged = context.is_prefill and context.block_tables is not None
         fold = have_cache and not kv_stored and (
             (self.k_scale is None and foldable(k, v))

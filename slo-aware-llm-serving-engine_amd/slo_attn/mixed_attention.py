@@ -44,20 +44,18 @@ def forward_mixed(q, k, v, k_cache, v_cache, context, scale, store_fn,
     meta = context.mixed
     if not k_cache.numel() or not v_cache.numel():
         raise RuntimeError("mixed forward requires an allocated KV pool")
-    # The library's own store runs inside the attention launch when the new
-    # rows are contiguous and the step has decode rows (same result, one
-    # launch less; a step of prefill rows that read the pool gets the store
-    # kernel first from the same call, so that its long rows can split their
-    # keys over 32-position blocks); any other store_fn runs first.  An E4M3FN
-    # pool folds it only into pure decode steps (with at most 8 query heads per
-    # kv head: the launch quantises each decode row's newest token itself) and
-    # steps of cold prefill rows, whose items quantise their own tokens.  With
-    # decode and prefill rows the folded E4M3FN launch measured slower than the
-    # store kernel and the launch: rows reading the pool re-quantise their new
+    # The library's own store runs inside the attention launch (same result, one
+    # launch less) for bf16 pools and contiguous new rows: with decode rows in
+    # the launch itself; a step of prefill rows that read the pool gets the
+    # store kernel first from the same call, so that its long rows can split
+    # their keys over 32-position blocks.  Pure decode steps, and steps of cold
+    # prefill rows only (they read no pool), also fold rows that are views of
+    # the QKV projection, and into E4M3FN pools (at most 8 query heads per kv
+    # head: the launch quantises the new tokens itself).  With decode and
+    # prefill rows the folded E4M3FN launch measured slower than the store
+    # kernel and the launch: rows reading the pool re-quantise their new
     # tokens' tiles in every item (24 decode rows and two chunks, one after a
-    # 1,024-token prefix: 108 against 72 us).
-    # Pure decode steps, and steps of cold prefill rows only (they read no
-    # pool), also fold rows that are views of the QKV projection.
+    # 1,024-token prefix: 108 against 72 us).  Any other store_fn runs first.
     alone = not meta.num_prefill_tokens or (not meta.num_decode and not meta.prefill_has_history)
     fold = (store_fn is store_kvcache and phases == _lib.PHASE_ALL
             and ((foldable(k, v)
