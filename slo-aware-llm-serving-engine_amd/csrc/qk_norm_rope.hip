@@ -21,12 +21,14 @@
 // One 512-thread workgroup per token; a 16-lane group per head of the QKV
 // row, lane j holding elements 8j..8j+7 (one 16-byte load), so a head's
 // statistics are a 16-lane reduction and the RoPE partner of element d
-// (d +- 64) sits in lane j ^ 8.  Bound by VALU issue at many tokens (28.5 MB
-// for 1,048 tokens are 5.6 us of a copy) and by one dependent chain of loads
-// at few: the sums reduce by DPP moves instead of LDS permutes, the fp64
-// square root and division are one refined v_rsq_f64, the sine is negated
-// once per token instead of choosing between two results per element, and
-// rows are addressed by a uniform base and a 32-bit offset: 9.6 -> 8.5 us for
+// (d +- 64) sits in lane j ^ 8.  Bound by VALU issue beside the traffic at many
+// tokens (1,048 tokens: 28.5 MB, 5.6 us of a copy; 255 VALU instructions a
+// wavefront, 8.2 wavefronts a SIMD, the fp64 ones at a quarter of the rate) and
+// by one dependent chain of loads at few.  The sums reduce by DPP moves instead
+// of LDS permutes, the fp64 square root and division are one refined
+// v_rsq_f64, the sine is negated once per token instead of choosing between
+// two results per element, and rows are addressed by a uniform base and a
+// 32-bit offset (320 -> 255 VALU instructions a wavefront): 9.6 -> 8.5 us for
 // 1,048 tokens, the same buffers replayed; 10.8 -> 10.1 us where each of 8
 // layers has its own, read from HBM.  (On the same buffers, 384 threads, two
 // heads in every group, 9.1 us; before these changes 256 threads and three
