@@ -10,7 +10,7 @@
 // through HBM instead of four.  Arithmetic follows the reference's rounding
 // points:
 //   RMSNorm  var = mean(x^2) in fp32 (here: the exact mean, rounded once),
-//            r = rsqrt(var + eps) in fp32 (here: correctly rounded),
+//            r = rsqrt(var + eps) in fp32 (here: rounded from an fp64 value),
 //            n = bf16(x * r), out = bf16(n * w)
 //   RoPE     x1, x2 = halves of out (as fp32); y1 = x1*cos - x2*sin,
 //            y2 = x2*cos + x1*sin, each product and sum rounded in fp32 (no
@@ -21,9 +21,9 @@
 // One 512-thread workgroup per token; a 16-lane group per head of the QKV
 // row, lane j holding elements 8j..8j+7 (one 16-byte load), so a head's
 // statistics are a 16-lane reduction and the RoPE partner of element d
-// (d +- 64) sits in lane j ^ 8.  Bound by VALU issue beside the traffic at many
-// tokens (1,048 tokens: 28.5 MB, 5.6 us of a copy; 255 VALU instructions a
-// wavefront, 8.2 wavefronts a SIMD, the fp64 ones at a quarter of the rate) and
+// (d +- 64) sits in lane j ^ 8.  Bound by the traffic and VALU issue that it
+// only partly overlaps at many tokens (1,048 tokens: 28.5 MB, 5.6 us of a copy;
+// 255 VALU instructions a wavefront, 8.2 wavefronts a SIMD, about 3.5 us) and
 // by one dependent chain of loads at few.  The sums reduce by DPP moves instead
 // of LDS permutes, the fp64 square root and division are one refined
 // v_rsq_f64, the sine is negated once per token instead of choosing between
